@@ -233,6 +233,30 @@ bool nonneg(const weft_ggml_tensor* t) {
   return true;
 }
 
+// decode_quantized's code of a src0 type (Q4_K: 8), and its two table arguments
+int gemv_format(int32_t type) {
+  switch (type) {
+    case WEFT_GGML_TYPE_Q4_0: return 0;
+    case WEFT_GGML_TYPE_MXFP4: return 1;
+    case WEFT_GGML_TYPE_IQ2_XXS: return 2;
+    case WEFT_GGML_TYPE_Q6_K: return 3;
+    case WEFT_GGML_TYPE_Q5_K: return 4;
+    case WEFT_GGML_TYPE_NVFP4: return 5;
+    case WEFT_GGML_TYPE_Q4_1: return 6;
+    case WEFT_GGML_TYPE_IQ2_XS: return 7;
+    default: return 8;
+  }
+}
+const int8_t* tables0(const GgmlTables* tab, int32_t type) {
+  if (tab == nullptr) return nullptr;
+  return type == WEFT_GGML_TYPE_IQ2_XXS ? tab->grid : type == WEFT_GGML_TYPE_IQ2_XS ? tab->grid_xs : tab->codebook;
+}
+const void* tables1(const GgmlTables* tab, int32_t type) {
+  if (tab == nullptr) return nullptr;
+  if (type == WEFT_GGML_TYPE_IQ2_XXS || type == WEFT_GGML_TYPE_IQ2_XS) return tab->signs;
+  return type == WEFT_GGML_TYPE_NVFP4 ? tab->ue4m3 : tab->scale;
+}
+
 hipError_t mul_mat(const weft_ggml_tensor* s0, const weft_ggml_tensor* s1, const weft_ggml_tensor* d,
                    void* wdata, size_t wsize) {
   if (s0 == nullptr || s1 == nullptr || d == nullptr) return fail(hipErrorInvalidValue);
@@ -315,6 +339,9 @@ hipError_t mul_mat(const weft_ggml_tensor* s0, const weft_ggml_tensor* s1, const
             break;
           default: mul_mat_mxfp4(W, X, Xq, tab->codebook, tab->scale, Y, n, k, m, st); break;
         }
+      } else if (small_batch_quantized(gemv_format(s0->type), W, src1, tables0(tab, s0->type), tables1(tab, s0->type), Y,
+                                       n, k, m, st)) {
+        // done: a few rows of an activation that is already quantized
       } else {
         switch (s0->type) {
           case WEFT_GGML_TYPE_Q4_0: decode_quantized(0, W, src1, nullptr, nullptr, Y, n, k, m, st); break;
@@ -403,40 +430,49 @@ hipError_t mul_mat_id(const weft_ggml_tensor* s0, const weft_ggml_tensor* s1,
   const uint8_t* xq_in = quantize ? nullptr : static_cast<const uint8_t*>(s1->data);
   uint8_t* xq_out = quantize ? static_cast<uint8_t*>(wdata) : nullptr;
   float* Y = static_cast<float*>(d->data);
+  // src1 rows (t, j) -> records at (t * ne11 + j) * nbw1 of wdata
+  auto quantize_rows = [&](void (*rows)(const float*, size_t, uint8_t*, size_t, size_t)) {
+    if (!quantize) return;
+    const size_t k = (size_t)K;
+    if (ne11 == 1) {
+      rows(X, n_tok > 1 ? (size_t)pr.x_s2 : k, xq_out, (size_t)n_tok, k);
+    } else if (n_tok == 1 || pr.x_s2 == (long long)ne11 * pr.x_s1) {
+      rows(X, (size_t)pr.x_s1, xq_out, (size_t)(ne11 * n_tok), k);
+    } else {
+      for (int64_t t = 0; t < n_tok; ++t)
+        rows(X + (size_t)t * pr.x_s2, (size_t)pr.x_s1, xq_out + (size_t)t * ne11 * nbw1, (size_t)ne11, k);
+    }
+  };
+  auto quantize_q8k = [&]() { quantize_rows(quantize_q8_k_rows); };
+  const uint8_t* xq = quantize ? xq_out : xq_in;
+  const bool grouped = n_pairs >= 64 && n_pairs >= 4 * n_as;
+  // a few pairs of several tokens: each expert's weights are read once for all
+  // of its pairs.  One token's pairs choose different experts, and their GEMV
+  // quantizes in the same launch.
+  const bool rows_apart = !quantize || (aligned(X, 4) && (ne11 == 1 ? pr.x_s2 : pr.x_s1) >= K);
+  if (!grouped && n_tok > 1 && rows_apart &&
+      small_pairs_ok(gemv_format(s0->type), W, xq, tables0(tab, s0->type), tables1(tab, s0->type), Y, (size_t)N,
+                     (size_t)K, st, pr, n_pairs, (size_t)(ne11 * n_tok))) {
+    quantize_rows(vd->size == kQ8_KBytes   ? quantize_q8_k_rows
+                  : vd->size == kQ8_1Bytes ? quantize_q8_1_rows
+                                           : quantize_q8_0_rows);
+    small_pairs(gemv_format(s0->type), W, xq, tables0(tab, s0->type), tables1(tab, s0->type), Y, (size_t)N, (size_t)K,
+                st, pr, n_pairs);
+    return pending_error();
+  }
   // several pairs per expert on average, or rows the pair GEMV cannot hold
   // in LDS: group the pairs by expert on the device and run the grouped MFMA
   // GEMM (GGML's own order: quantize src1, group, multiply); the grouping
   // lives in the part of wdata GGML's plan reserves for its row mapping
-  const int gemv_fmt = s0->type == WEFT_GGML_TYPE_Q4_0     ? 0
-                       : s0->type == WEFT_GGML_TYPE_MXFP4   ? 1
-                       : s0->type == WEFT_GGML_TYPE_IQ2_XXS ? 2
-                       : s0->type == WEFT_GGML_TYPE_Q6_K    ? 3
-                       : s0->type == WEFT_GGML_TYPE_Q5_K    ? 4
-                       : s0->type == WEFT_GGML_TYPE_NVFP4   ? 5
-                       : s0->type == WEFT_GGML_TYPE_Q4_1    ? 6
-                                                            : 7;
+  const int gemv_fmt = gemv_format(s0->type);
   const bool pair_gemv_fits = s0->type == WEFT_GGML_TYPE_Q4_K ? q4k_gemv_fits((size_t)K)
                                                               : staged_gemv_fits(gemv_fmt, (size_t)K);
-  if (((n_pairs >= 64 && n_pairs >= 4 * n_as) || !pair_gemv_fits) && wdata != nullptr) {
+  if ((grouped || !pair_gemv_fits) && wdata != nullptr) {
     const size_t xq_bytes = nbw1 * (size_t)(ne11 * n_tok);
     const size_t used = quantize ? (xq_bytes + 15) & ~(size_t)15 : 0;
     uint8_t* ws = static_cast<uint8_t*>(wdata) + used;
     const size_t ws_bytes = wsize >= used ? wsize - used : 0;
     const size_t n = (size_t)N, k = (size_t)K;
-    // src1 rows (t, j) -> Q8_K records at (t * ne11 + j) * nbw1 of wdata
-    auto quantize_q8k = [&]() {
-      if (!quantize) return;
-      if (ne11 == 1) {
-        quantize_q8_k_rows(X, n_tok > 1 ? (size_t)pr.x_s2 : k, xq_out, (size_t)n_tok, k);
-      } else if (n_tok == 1 || pr.x_s2 == (long long)ne11 * pr.x_s1) {
-        quantize_q8_k_rows(X, (size_t)pr.x_s1, xq_out, (size_t)(ne11 * n_tok), k);
-      } else {
-        for (int64_t t = 0; t < n_tok; ++t)
-          quantize_q8_k_rows(X + (size_t)t * pr.x_s2, (size_t)pr.x_s1, xq_out + (size_t)t * ne11 * nbw1,
-                             (size_t)ne11, k);
-      }
-    };
-    const uint8_t* xq = quantize ? xq_out : xq_in;
     switch (s0->type) {
       case WEFT_GGML_TYPE_Q4_K:
         if (mul_mat_id_q4k_grouped_ok(W, xq_bytes, Y, n, k, st, pr, n_pairs, ws, ws_bytes)) {

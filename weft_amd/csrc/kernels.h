@@ -214,6 +214,25 @@ bool mul_mat_id_kq_grouped_ok(bool q6, const uint8_t* W, size_t xq_bytes, const 
 void mul_mat_id_kq_grouped(bool q6, const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K,
                            const RowStrides& st, const PairArgs& pr, int n_pairs, void* ws);
 
+// Small-batch mul_mat (small_batch.hip): 2 .. kSmallBatchRows activation rows
+// on one 16-row-wide MFMA GEMM whose waves split K, any format (decode_quantized's
+// codes, Q4_K = 8), record alignment and K.  X is quantized into Xq; _quantized
+// reads Xq.  False, with nothing launched, when the call does not suit it.
+constexpr size_t kSmallBatchRows = 64;
+bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* tab0, const void* tab1,
+                 float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
+bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
+                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
+
+// MUL_MAT_ID's (token, slot) pairs on the same kernel, 2 .. 64 of them, which
+// groups them by expert itself: Xq holds the x_rows quantized src1 rows
+// (token * ne11 + row).  _ok: whether the shape suits it.
+bool small_pairs_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
+                    const float* Y, size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs,
+                    size_t x_rows);
+void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1, float* Y,
+                 size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs);
+
 // Activation quantizers over K contiguous values, and over M rows of K
 // values ldx floats apart (records written contiguously).
 void quantize_q8_k(const float* X, uint8_t* Y, size_t K);

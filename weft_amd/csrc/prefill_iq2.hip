@@ -480,6 +480,7 @@ bool gemm_iq2_try(bool xs, const uint8_t* W, const float* X, uint8_t* Xq, const 
 void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid,
                      const int8_t* signs, float* Y, size_t N, size_t K, size_t M,
                      const RowStrides& st) {
+  if (small_batch(2, W, X, Xq, grid, signs, Y, N, K, M, st)) return;
   if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok(W, Xq, Y, grid, signs, N, K, M, st))
     return decode_iq2_xxs(W, X, Xq, grid, signs, Y, N, K, M, st);
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);
@@ -489,6 +490,7 @@ void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t
 // IQ2_XS: the same GEMM with per-half scales (M >= 16, K % 512 == 0), the GEMV otherwise
 void mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid, const int8_t* signs,
                     float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
+  if (small_batch(7, W, X, Xq, grid, signs, Y, N, K, M, st)) return;
   if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok<true>(W, Xq, Y, grid, signs, N, K, M, st))
     return decode_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, st);
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);

@@ -621,6 +621,7 @@ bool gemm_q4k_try(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
 void mul_mat_q4k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                  size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return;
+  if (small_batch(8, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
   // the GEMV below 16 activation rows, unless its LDS cannot hold a row
   if ((M >= 16 || !q4k_gemv_fits(K)) && X != nullptr && args_ok(W, Xq, Y, N, K, M, st) &&
       gemm_q4k_ok(W, N, K, M, st)) {

@@ -1134,6 +1134,7 @@ bool gemm_q80_try(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const 
 void mul_mat_q4_0(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                   size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return decode_q4_0(W, X, Xq, Y, N, K, M, st);
+  if (small_batch(0, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
       !prefill_q80<WFmt::Q4_0>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st))
     decode_q4_0(W, X, Xq, Y, N, K, M, st);
@@ -1142,6 +1143,7 @@ void mul_mat_q4_0(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
 void mul_mat_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                   size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return decode_q4_1(W, X, Xq, Y, N, K, M, st);
+  if (small_batch(6, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
       !prefill_q80<WFmt::Q4_1>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st))
     decode_q4_1(W, X, Xq, Y, N, K, M, st);
@@ -1150,6 +1152,7 @@ void mul_mat_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
 void mul_mat_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                    const float* ue4m3, float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return decode_nvfp4(W, X, Xq, codebook, ue4m3, Y, N, K, M, st);
+  if (small_batch(5, W, X, Xq, codebook, ue4m3, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
       !prefill_q80<WFmt::NVFP4>(W, X, Xq, codebook, ue4m3, Y, N, K, M, st))
     decode_nvfp4(W, X, Xq, codebook, ue4m3, Y, N, K, M, st);
@@ -1158,6 +1161,7 @@ void mul_mat_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* 
 void mul_mat_mxfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                    const float* scale, float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return decode_mxfp4(W, X, Xq, codebook, scale, Y, N, K, M, st);
+  if (small_batch(1, W, X, Xq, codebook, scale, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
       !prefill_q80<WFmt::MXFP4>(W, X, Xq, codebook, scale, Y, N, K, M, st))
     decode_mxfp4(W, X, Xq, codebook, scale, Y, N, K, M, st);
