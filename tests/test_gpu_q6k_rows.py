@@ -1,0 +1,57 @@
+"""Q6_K prefill GEMM on weight rows that are only 2-byte aligned (an odd number
+of 210-byte records a row, a 2-byte offset or row pad), dense and grouped
+(MUL_MAT_ID), against the oracle, and extreme scales: its weight operands are
+two int8 digits of scale x value, up to 128 x 32."""
+import numpy as np
+import pytest
+
+import oracle as o
+from weft_amd import ggml as G
+from .test_gpu_ggml import run, run_id
+
+pytestmark = pytest.mark.gpu
+
+
+def launched(call):
+    from weft_amd import _lib
+    _lib.launch_log()
+    call()
+    return _lib.launch_log()
+
+
+@pytest.mark.parametrize("superblocks,n,m,pad", [
+    (1, 130, 65, 0), (3, 300, 80, 0), (43, 75, 129, 0),  # odd superblock counts, ragged tiles
+    (2, 130, 65, 2), (4, 64, 70, 6),                     # whole pairs, rows 2 bytes off
+])
+def test_two_byte_rows(hip, superblocks, n, m, pad):
+    names = launched(lambda: run(hip, "q6_k", 256 * superblocks, n, m, pad_w=pad, pad_x=4, pad_y=4))
+    assert "q6k_mfma_gemm" in names, names
+
+
+@pytest.mark.parametrize("superblocks,pad", [(3, 0), (2, 2), (2, 4)])
+def test_two_byte_rows_grouped(hip, superblocks, pad):
+    ids = np.random.default_rng(9).integers(0, 5, size=(60, 2))
+    names = launched(lambda: run_id(hip, "q6_k", 256 * superblocks, 150, 5, 2, 1, 60, ids, pad_w=pad))
+    assert "q6k_mfma_gemm" in names, names
+
+
+@pytest.mark.parametrize("superblocks", [1, 2, 5])
+def test_extreme_scales(hip, superblocks):
+    """Every 16-group scale at -128, -127, 127 or 0 and values at both ends of
+    the 6-bit range against activations of +-127."""
+    rng = np.random.default_rng(12)
+    n, k, m = 96, 256 * superblocks, 70
+    w = o.random_records("q6_k", n, k, seed=13).reshape(n, superblocks, 210)
+    w[:, :, :192] = rng.choice(np.array([0, 255], np.uint8), size=(n, superblocks, 192))
+    w[:, :, 192:208] = rng.choice(np.array([128, 129, 127, 0], np.uint8), size=(n, superblocks, 16))
+    w[:, :, 208:210] = np.full((n, superblocks, 1), 3e-4, np.float16).view(np.uint8)
+    w = np.ascontiguousarray(w.reshape(n, -1))
+    x = rng.choice(np.array([-1.0, 1.0, 0.5], np.float32), size=(m, k)).astype(np.float32)
+    xq = o.quantize("q8_k", x)
+    e, a = o.mul_mat_f64("q6_k", w, xq, n, k, m)
+    wd, xd, yd = hip.to_dev(w), hip.to_dev(x), hip.empty(4 * n * m)
+    s0, s1 = G.tensor(G.Q6_K, (k, n), wd.ptr), G.tensor(G.F32, (k, m), xd.ptr)
+    work = hip.empty(G.mul_mat_work_size(s0, s1))
+    G.mul_mat(s0, s1, G.tensor(G.F32, (n, m), yd.ptr), work.ptr, work.nbytes)
+    hip.torch.cuda.synchronize()
+    assert o.within_tolerance(yd.numpy(np.float32).reshape(m, n), e, a).all()

@@ -5,13 +5,18 @@
 // Q6_K (ggml-cpu/quants.c:800-853):
 //   Y[m,n] = sum_b (dw[n,b] dx[m,b]) * sum_{j<16} sc[n,b,j] * P[m,n,b,j]
 //   P = sum_{k in 16-group j} q8[m,k] * (q6[n,k] - 32)                (exact int32)
-// The signed 8-bit scale times a 6-bit value does not fit an int8 operand,
-// so it is applied after the product: one v_mfma_i32_32x32x32_i8 covers a
-// 32-group, and it runs twice with the weight operand of one 16-element half
-// (the lanes of the other half hold zeros); each product tile takes its
-// half's scale in one v_mad_i32_i24 per output (|P| <= 65536, |sc| <= 128,
-// eight groups < 2^27).  The weight operand is q6 - 32 as a signed byte,
-// formed four at a time: ((q | 0x80) - 0x20) ^ 0x80 never borrows.
+// The signed 8-bit scale times the 6-bit value, p = sc (q6 - 32), does not fit
+// an int8 operand (|p| <= 4096), but it is two of them exactly, p = 256 H + L
+// with L its signed low byte: two v_mfma_i32_32x32x32_i8 per 32-group, whose
+// int32 tiles run over the half superblock, S = lo + 256 hi.  Lane half kg of
+// the operand holds exactly the 16 elements of scale group 2 s + kg, so a
+// lane multiplies by one scale: v_pk_mad_u16 gives p + 128 for two values, of
+// which a byte permute takes the high bytes (H) and the low ones (L + 128).
+// What bounds it is VALU issue beside the MFMAs: about 11 instructions per
+// four weights and 3 per output and half superblock.  Before, each 16-group's
+// product tile took its scale on VALU (two masked MFMAs per 32-group and two
+// multiply-adds per output): 633 VALU instructions per wave and half
+// superblock, now about 300.
 //
 // Q5_K (ggml-cpu/quants.c:720-798):
 //   Y[m,n] = sum_b (dw dx) * S - (dmin dx) * Mn
@@ -36,9 +41,12 @@
 // global->LDS loads while computing b (Q5_K's 176-byte records as 16-byte
 // chunks when the rows are aligned).  A Q6_K record (210 bytes) is 2-byte
 // aligned for odd b, so its row is staged from the dword holding its first
-// byte (54 dwords, 216 bytes per LDS row) and the odd superblocks read with
+// byte (53 dwords as 16-byte chunks, 240 bytes per LDS row: 16 lanes' reads
+// fall on all 64 banks) and the odd superblocks read with
 // a 2-byte alignment; the even/odd slots are the two instantiations of the
-// step.  Both halves' partial sums meet in LDS at the end and every output
+// step.  Rows that are themselves only 2-byte aligned (an odd number of
+// superblocks) take the third, which aligns by each lane's own row.  Both
+// halves' partial sums meet in LDS at the end and every output
 // is written once, even + odd, with 16-byte stores (tile_store.h).
 #include <algorithm>
 #include <type_traits>
@@ -56,6 +64,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef short v2s __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
@@ -70,12 +79,12 @@ template <KQ F>
 struct KTile {
   static constexpr bool k6 = F == KQ::Q6_K;
   static constexpr int kRec = k6 ? kQ6_KBytes : kQ5_KBytes;  // 210 / 176
-  static constexpr int kLoadD = k6 ? 54 : 44;                // dwords staged per weight row
-  static constexpr int kRowB = 4 * kLoadD;                   // LDS bytes per weight row: 216 / 176
+  static constexpr int kRowB = k6 ? 240 : 176;               // LDS bytes per weight row
+  static constexpr int kLoadD = kRowB / 4;                   // in dwords
   static constexpr int kBS = k6 ? 0 : kMT * 32;              // Q5_K: the tokens' bsums
   static constexpr int kWT = kNT * kRowB;
-  static constexpr int kSlot = kAQ + kBS + kWT;              // 44,032 / 40,960
-  static constexpr int kWSlots = kNT * kLoadD / 64;          // 108 / 88 wave-wide dword loads
+  static constexpr int kSlot = kAQ + kBS + kWT;              // 47,104 / 40,960
+  static constexpr int kWSlots = kNT * kLoadD / 64;          // wave-wide dword loads (Q5_K: 88)
   static_assert(kNT * kLoadD % 64 == 0, "weight tile is whole wave loads");
   static_assert(kTilePlaneBytes <= kSlot, "an output plane fits one ring slot");
 };
@@ -110,21 +119,23 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 }
 __device__ __forceinline__ void pin(int& v) { asm volatile("" : "+v"(v)); }
 
-// 16 bytes that start kSh (0 or 2) bytes past the 8-byte aligned LDS address p
+// 16 bytes that start sh (0 or 2) bytes past the 16-byte aligned LDS address
+// p: kSh = sh where it is known, else kRowShift
+constexpr int kRowShift = -1;
 template <int kSh>
-__device__ __forceinline__ uint4 ld16(const uint8_t* p) {
-  const uint2 a = *reinterpret_cast<const uint2*>(p);
-  const uint2 b = *reinterpret_cast<const uint2*>(p + 8);
+__device__ __forceinline__ uint4 ld16(const uint8_t* p, uint32_t sh) {
+  const uint4 a = *reinterpret_cast<const uint4*>(p);
   if constexpr (kSh == 0) {
-    return make_uint4(a.x, a.y, b.x, b.y);
+    return a;
   } else {
     const uint32_t c = *reinterpret_cast<const uint32_t*>(p + 16);
-    return make_uint4(__builtin_amdgcn_alignbyte(a.y, a.x, kSh), __builtin_amdgcn_alignbyte(b.x, a.y, kSh),
-                      __builtin_amdgcn_alignbyte(b.y, b.x, kSh), __builtin_amdgcn_alignbyte(c, b.y, kSh));
+    return make_uint4(__builtin_amdgcn_alignbyte(a.y, a.x, sh), __builtin_amdgcn_alignbyte(a.z, a.y, sh),
+                      __builtin_amdgcn_alignbyte(a.w, a.z, sh), __builtin_amdgcn_alignbyte(c, a.w, sh));
   }
 }
 
-template <bool kGroup, KQ F>
+// kOdd (Q6_K): weight rows that are only 2-byte aligned
+template <bool kGroup, KQ F, bool kOdd = false>
 __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
   using TT = KTile<F>;
   constexpr bool k6 = TT::k6;
@@ -195,9 +206,24 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
       if (wave < 2) lds_dma16(bsrc + (size_t)b * kQ8_KBytes, base + kAQ + 1024 * wave);
     }
     // weight rows: Q6_K from the dword holding the record's first byte (2
-    // bytes before it for odd b); dword 53 is padding and re-reads dword 52
-    const size_t wb = (size_t)b * TT::kRec - (k6 ? 2 * (b & 1) : 0);
-    if constexpr (!k6) {
+    // bytes before it for odd b), 53 dwords
+    const size_t wb = (size_t)b * TT::kRec - (k6 && !kOdd ? 2 * (b & 1) : 0);
+    if constexpr (k6) {
+      // 15 chunks of 16 bytes a row (30 wave-wide loads, the row q / 15): 0 ..
+      // 12 in place, 13 and 14 both the 16 bytes that end with dword 52, which
+      // so lands at bytes 220 .. 223 and nothing past it is read
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = wave + 8 * i;
+        if (k < kNT * 15 / 64) {
+          const int q = 64 * k + lane, row = q / 15, c = q - 15 * row;
+          const uint8_t* g = W + (size_t)min(n0 + row, a.N - 1) * wrb + wb;
+          if constexpr (kOdd) g -= (uint32_t)(uintptr_t)g & 2u;
+          lds_dma16(g + min(16 * c, 196), base + kAQ + TT::kBS + 1024 * k);
+        }
+      }
+      return;
+    } else {
       // Q5_K records are 11 chunks of 16 bytes: 22 wave-wide 16-byte loads
       // when the rows are 16-byte aligned (row q / 11, chunk q % 11)
       if (w16) {
@@ -218,7 +244,7 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
       const int k = wave + 8 * i;
       if (k < kWSlots) {
         const int q = 64 * k + lane, row = q / kLoadD, part = q - kLoadD * row;
-        const uint8_t* g = W + (size_t)min(n0 + row, a.N - 1) * wrb + wb + 4 * (k6 ? min(part, 52) : part);
+        const uint8_t* g = W + (size_t)min(n0 + row, a.N - 1) * wrb + wb + 4 * part;
         lds_dma4(g, base + kAQ + TT::kBS + 256 * k);
       }
     }
@@ -226,7 +252,7 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
   float dxr = 0.f;
   auto load_dx = [&](int b) { dxr = *reinterpret_cast<const float*>(dsrc + (size_t)b * kQ8_KBytes); };
 
-  v16i acc[2];
+  v16i acc[2], hi[2];
   v16f y[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -234,9 +260,12 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     for (int r = 0; r < 16; ++r) y[t][r] = 0.f;
   const v16i zero = {};
   const int sw = col & 15;
+  // (kOdd) the low address bits of this lane's weight row
+  const uint32_t row_addr = (uint32_t)(uintptr_t)(W + (size_t)min(n0 + 32 * wcol + col, a.N - 1) * wrb);
 
   auto step = [&](int b, const uint8_t* cur, int nxt, auto shift) {
     constexpr int kSh = decltype(shift)::value;  // byte offset of the Q6_K record in its LDS row
+    const uint32_t sh = kSh == kRowShift ? (uint32_t)(row_addr + (uint32_t)b * TT::kRec) & 2u : (uint32_t)kSh;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of superblock b have landed
     __syncthreads();                // everyone's; superblock b - 1 is consumed
     const bool refill = b + 1 < nsb;
@@ -252,48 +281,44 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     v16f mn[2];
     if constexpr (k6) {
       // ql of groups s = 0, 2 (P0) and 1, 3 (P1), qh of all four, the 8 scales of the half
-      const uint4 P0 = ld16<kSh>(row + 64 * h + 16 * kg);
-      const uint4 P1 = ld16<kSh>(row + 64 * h + 32 + 16 * kg);
-      const uint4 Q = ld16<kSh>(row + 128 + 32 * h + 16 * kg);
+      const uint4 P0 = ld16<kSh>(row + 64 * h + 16 * kg, sh);
+      const uint4 P1 = ld16<kSh>(row + 64 * h + 32 + 16 * kg, sh);
+      const uint4 Q = ld16<kSh>(row + 128 + 32 * h + 16 * kg, sh);
       const uint2 s8 = *reinterpret_cast<const uint2*>(row + 192 + 8 * h);
       uint32_t sc0 = s8.x, sc1 = s8.y;
       if constexpr (kSh != 0) {
-        const uint32_t s2 = *reinterpret_cast<const uint32_t*>(row + 200 + 8 * h);
-        sc0 = __builtin_amdgcn_alignbyte(s8.y, s8.x, kSh);
-        sc1 = __builtin_amdgcn_alignbyte(s2, s8.y, kSh);
+        const uint32_t s2 = *reinterpret_cast<const uint32_t*>(row + 200 + 20 * h);  // dword 50 or 52
+        sc0 = __builtin_amdgcn_alignbyte(s8.y, s8.x, sh);
+        sc1 = __builtin_amdgcn_alignbyte(s2, s8.y, sh);
       }
-      const uint32_t dword = *reinterpret_cast<const uint32_t*>(row + 208);
-      dw = fp16_to_fp32(kSh ? dword >> 16 : dword & 0xffffu);
+      const uint32_t dword = *reinterpret_cast<const uint32_t*>(row + 220);
+      dw = fp16_to_fp32((dword >> (8 * sh)) & 0xffffu);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const uint4 L = (s & 1) ? P1 : P0;
         const uint32_t lq[4] = {L.x, L.y, L.z, L.w}, hq[4] = {Q.x, Q.y, Q.z, Q.w};
-        v4i bv;
+        // this lane's 16 elements have one scale: 2 s + kg of the half
+        const short sc = (short)(int8_t)((s < 2 ? sc0 : sc1) >> (16 * (s & 1) + 8 * kg));
+        const v2s m = {sc, sc}, c = {(short)(128 - 32 * sc), (short)(128 - 32 * sc)};
+        v4i lo_w, hi_w;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const uint32_t lo = ((lq[i] >> (4 * (s >> 1))) & 0x0f0f0f0fu) | 0x80808080u;
-          const uint32_t hi = (s < 3 ? hq[i] << (4 - 2 * s) : hq[i] >> 2) & 0x30303030u;
-          bv[i] = (int)(((lo | hi) - 0x20202020u) ^ 0x80808080u);  // q6 - 32, four signed bytes
+          const uint32_t q = ((lq[i] >> (4 * (s >> 1))) & 0x0f0f0f0fu) |
+                             ((s < 3 ? hq[i] << (4 - 2 * s) : hq[i] >> 2) & 0x30303030u);
+          // p + 128 of values 0, 2 and of 1, 3 (p = sc (q - 32), 16 bits)
+          const v2s te = __builtin_bit_cast(v2s, q & 0x00ff00ffu) * m + c;
+          const v2s to = __builtin_bit_cast(v2s, __builtin_amdgcn_perm(0u, q, 0x0c030c01u)) * m + c;
+          const uint32_t ue = __builtin_bit_cast(uint32_t, te), uo = __builtin_bit_cast(uint32_t, to);
+          lo_w[i] = (int)(__builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u);
+          hi_w[i] = (int)__builtin_amdgcn_perm(uo, ue, 0x07030501u);
         }
-        const v4i bz = {};
-        const uint32_t sb = ((s < 2 ? sc0 : sc1) >> (16 * (s & 1))) & 0xffffu;
-        const int sc_lo = (int)(int8_t)(sb & 0xffu), sc_hi = (int)(int8_t)(sb >> 8);
         const int chunk = (2 * (4 * h + s) + kg) ^ sw;
-        v16i I[2], I2[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const v4i av = *reinterpret_cast<const v4i*>(AQ + (32 * t + col) * 256 + 16 * chunk);
-          I[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, kg ? bz : bv, zero, 0, 0, 0);
-          I2[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, kg ? bv : bz, zero, 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, lo_w, s == 0 ? zero : acc[t], 0, 0, 0);
+          hi[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, hi_w, s == 0 ? zero : hi[t], 0, 0, 0);
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            int v = __mul24(I[t][r], sc_lo) + __mul24(I2[t][r], sc_hi) + (s == 0 ? 0 : acc[t][r]);
-            pin(v);
-            acc[t][r] = v;
-          }
         if (s == 1 && refill) issue(b + 1, nxt);
       }
     } else {
@@ -368,7 +393,7 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
                                                              __builtin_bit_cast(v8bf, bw), fz, 0, 0, 0);
       if constexpr (k6) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[t][r] = fmaf(qw[r], (float)acc[t][r], y[t][r]);
+        for (int r = 0; r < 16; ++r) y[t][r] = fmaf(qw[r], (float)(acc[t][r] + 256 * hi[t][r]), y[t][r]);
       } else {
         const v16f qm = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, aq),
                                                                __builtin_bit_cast(v8bf, bm), fz, 0, 0, 0);
@@ -385,8 +410,8 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     dxq[0][lane] = bf16_split3(dxr);
   }
   for (int b = 0; b < nsb; b += 2) {
-    step(b, ring0, 1, std::integral_constant<int, 0>{});
-    if (b + 1 < nsb) step(b + 1, ring1, 0, std::integral_constant<int, k6 ? 2 : 0>{});
+    step(b, ring0, 1, std::integral_constant<int, kOdd ? kRowShift : 0>{});
+    if (b + 1 < nsb) step(b + 1, ring1, 0, std::integral_constant<int, kOdd ? kRowShift : k6 ? 2 : 0>{});
   }
 
   // both parities' partial sums -> two LDS planes (reusing the ring) -> Y
@@ -403,19 +428,24 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
       [](float e, float o) { return e + o; });
 }
 
-// MFMA path: prefill shapes with 4-byte aligned weight rows; Q6_K also needs
-// an even number of superblocks per row (its odd records start 2 bytes into
-// a dword).  The GEMV kernels take everything else.
+// MFMA path: prefill shapes with 4-byte aligned weight rows, Q6_K also with
+// 2-byte aligned ones (kq_odd: a row of an odd number of 210-byte records
+// leaves the next one there).  The GEMV kernels take everything else.
+template <KQ F>
+bool kq_odd(const uint8_t* W, size_t ldw, size_t w_es, size_t K) {
+  return F == KQ::Q6_K && (K % 512 != 0 || !aligned(W, 4) || ldw % 4 != 0 || w_es % 4 != 0);
+}
+
 template <KQ F>
 bool gemm_kq_ok(const uint8_t* W, const void* Xq, const float* Y, size_t N, size_t K, size_t M,
                 const RowStrides& st) {
   constexpr size_t kRec = KTile<F>::kRec;
+  constexpr size_t kAlign = F == KQ::Q6_K ? 2 : 4;
   const size_t ldw = N > 1 ? st.ldw : K / 256 * kRec;
-  const size_t kq = F == KQ::Q6_K ? 512 : 256;
   // below 16 activation rows only when the GEMV's LDS cannot hold a row
-  return (M >= 16 || !staged_gemv_fits(F == KQ::Q6_K ? 3 : 4, K)) && N > 0 && K > 0 && K % kq == 0 &&
+  return (M >= 16 || !staged_gemv_fits(F == KQ::Q6_K ? 3 : 4, K)) && N > 0 && K > 0 && K % 256 == 0 &&
          W != nullptr && Xq != nullptr && Y != nullptr &&
-         aligned(W, 4) && ldw % 4 == 0 && aligned(Xq, 4) && aligned(Y, 4) && N <= (size_t)INT32_MAX &&
+         aligned(W, kAlign) && ldw % kAlign == 0 && aligned(Xq, 4) && aligned(Y, 4) && N <= (size_t)INT32_MAX &&
          K <= (size_t)INT32_MAX && M <= (size_t)INT32_MAX && strides_ok(st, K / 256 * kRec, 2, K, N, N, M) &&
          ((N + kNT - 1) / kNT) * ((M + kMT - 1) / kMT) <= (size_t)INT32_MAX;
 }
@@ -425,7 +455,10 @@ void gemm_kq(const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K, 
   const size_t ldw = N > 1 ? st.ldw : K / 256 * KTile<F>::kRec;
   GemmArgs ga{W, Xq, Y, (int)N, (int)K, (int)M, ldw, (long long)st.ldy, GroupTiles{}};
   const size_t tiles = ((N + kNT - 1) / kNT) * ((M + kMT - 1) / kMT);
-  kq_mfma_gemm<false, F><<<dim3((unsigned)tiles), kThreads, 0, current_stream()>>>(ga);
+  if (kq_odd<F>(W, ldw, 0, K))
+    kq_mfma_gemm<false, F, F == KQ::Q6_K><<<dim3((unsigned)tiles), kThreads, 0, current_stream()>>>(ga);
+  else
+    kq_mfma_gemm<false, F><<<dim3((unsigned)tiles), kThreads, 0, current_stream()>>>(ga);
   check_launch(F == KQ::Q6_K ? "q6k_mfma_gemm" : "q5k_mfma_gemm");
 }
 
@@ -483,9 +516,10 @@ bool mul_mat_id_kq_grouped_ok(bool q6, const uint8_t* W, size_t xq_bytes, const 
                               size_t ws_bytes) {
   const size_t rb = K / 256 * (q6 ? kQ6_KBytes : kQ5_KBytes);
   const size_t ldw = N > 1 ? st.ldw : rb;
-  return N > 0 && n_pairs > 0 && K > 0 && K % (q6 ? 512 : 256) == 0 && W != nullptr && Y != nullptr &&
-         aligned(W, 4) && ldw % 4 == 0 && aligned(Y, 4) && xq_bytes < ((size_t)1 << 32) && aligned(ws, 16) &&
-         ws_bytes >= moe_group_bytes(n_pairs, pr.n_as) && pr.w_es % 4 == 0 && pr.n_as <= kMaxExperts &&
+  const size_t align = q6 ? 2 : 4;
+  return N > 0 && n_pairs > 0 && K > 0 && K % 256 == 0 && W != nullptr && Y != nullptr &&
+         aligned(W, align) && ldw % align == 0 && aligned(Y, 4) && xq_bytes < ((size_t)1 << 32) && aligned(ws, 16) &&
+         ws_bytes >= moe_group_bytes(n_pairs, pr.n_as) && pr.w_es % (long long)align == 0 && pr.n_as <= kMaxExperts &&
          N <= (size_t)INT32_MAX && K <= (size_t)INT32_MAX && strides_ok(st, rb, 2, K, N, N, 1) &&
          (size_t)moe_tile_bound(n_pairs, pr.n_as) * ((N + kNT - 1) / kNT) <= (size_t)INT32_MAX;
 }
@@ -497,7 +531,10 @@ void mul_mat_id_kq_grouped(bool q6, const uint8_t* W, const uint8_t* Xq, float* 
   GemmArgs ga{W, Xq, Y, (int)N, (int)K, kMT, ldw, 0, group_tiles(g, pr)};
   const size_t wgs = (size_t)g.tmax * ((N + kNT - 1) / kNT);
   if (q6) {
-    kq_mfma_gemm<true, KQ::Q6_K><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
+    if (kq_odd<KQ::Q6_K>(W, ldw, (size_t)pr.w_es, K))
+      kq_mfma_gemm<true, KQ::Q6_K, true><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
+    else
+      kq_mfma_gemm<true, KQ::Q6_K><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
     check_launch("q6k_mfma_gemm");
   } else {
     kq_mfma_gemm<true, KQ::Q5_K><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
