@@ -36,6 +36,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef short v2s __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
@@ -134,10 +135,11 @@ __device__ __forceinline__ v4i weight_bytes(uint2 g0, uint2 g1, uint2 z0, uint2 
 
 // kXs (IQ2_XS, ggml-cpu/quants.c:897-946): u16 entries (grid row bits 0-8,
 // sign row bits 9-15) and a 4-bit scale per 16-element half, s_lo for
-// entries 0-1 and s_hi for 2-3 of each 32-group (scale byte 66 + g).  A
-// 32-group's MFMA runs twice with the weight operand of one half (the lanes
-// kg of the other half hold zeros), and each product tile takes its half's
-// 2 s + 1 in the same exact int32 multiply-add.
+// entries 0-1 and s_hi for 2-3 of each 32-group (scale byte 66 + g).  A lane
+// holds 16 elements of one half, so it multiplies its weights by that half's
+// 2 s + 1 (|p| <= 3968) and two MFMAs take p's signed byte digits, as in the
+// Q6_K GEMM: the int32 tiles run over the superblock, lo + 256 hi.  (Scales
+// on the product tiles took two masked MFMAs and 64 multiply-adds a group.)
 template <bool kGroup, bool kXs = false>
 __global__ void __launch_bounds__(kThreads, 1) iq2_mfma_gemm(GemmArgs a) {
   using TT = Tile<kXs>;
@@ -291,24 +293,28 @@ __global__ void __launch_bounds__(kThreads, 1) iq2_mfma_gemm(GemmArgs a) {
           const uint2 z0 = *reinterpret_cast<const uint2*>(tsg + 8 * (e0 >> 9));
           const uint2 z1 = *reinterpret_cast<const uint2*>(tsg + 8 * (e1 >> 9));
           const v4i bv = weight_bytes(g0, g1, z0, z1, canon);
-          const v4i bz = {};
-          const uint32_t sb = ((g < 4 ? scl0 : scl1) >> (8 * (g & 3))) & 0xffu;
-          const int ls_lo = 2 * (int)(sb & 15u) + 1, ls_hi = 2 * (int)(sb >> 4) + 1;
+          // this lane's 16 elements have one scale: p = (2 s + 1) w as two
+          // signed byte digits, p = 256 H + L
+          const uint32_t sb = ((g < 4 ? scl0 : scl1) >> (8 * (g & 3) + 4 * kg)) & 15u;
+          const short ls = (short)(2 * sb + 1);
+          const v2s m = {ls, ls}, c = {(short)(128 - 128 * ls), (short)(128 - 128 * ls)};
+          v4i lo_w, hi_w;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t u = (uint32_t)bv[i] ^ 0x80808080u;  // w + 128
+            const v2s te = __builtin_bit_cast(v2s, u & 0x00ff00ffu) * m + c;  // p + 128
+            const v2s to = __builtin_bit_cast(v2s, __builtin_amdgcn_perm(0u, u, 0x0c030c01u)) * m + c;
+            const uint32_t ue = __builtin_bit_cast(uint32_t, te), uo = __builtin_bit_cast(uint32_t, to);
+            lo_w[i] = (int)(__builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u);
+            hi_w[i] = (int)__builtin_amdgcn_perm(uo, ue, 0x07030501u);
+          }
           const int chunk = (2 * g + kg) ^ sw;
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const v4i av = *reinterpret_cast<const v4i*>(AQ + (32 * t + col) * 256 + 16 * chunk);
-            I[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, kg ? bz : bv, zero, 0, 0, 0);
-            I2[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, kg ? bv : bz, zero, 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, lo_w, g == 0 ? zero : acc[t], 0, 0, 0);
+            I2[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, hi_w, g == 0 ? zero : I2[t], 0, 0, 0);
           }
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              int v = __mul24(I[t][r], ls_lo) + __mul24(I2[t][r], ls_hi) + (g == 0 ? 0 : acc[t][r]);
-              pin(v);
-              acc[t][r] = v;
-            }
           continue;
         }
         const uint32_t w0 = wq[2 * g], w1 = wq[2 * g + 1], w2 = wq[2 * g + 2];
@@ -357,7 +363,10 @@ __global__ void __launch_bounds__(kThreads, 1) iq2_mfma_gemm(GemmArgs a) {
       const v16f qw = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, aq),
                                                              __builtin_bit_cast(v8bf, bw), fz, 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) y[t][r] = fmaf(qw[r], (float)acc[t][r], y[t][r]);
+      for (int r = 0; r < 16; ++r) {
+        const int S = kXs ? acc[t][r] + 256 * I2[t][r] : acc[t][r];
+        y[t][r] = fmaf(qw[r], (float)S, y[t][r]);
+      }
     }
     if (refill && wcol == 0) dxq[(pair + 1) & 1][par][lane] = bf16_split3(dxr);  // slot last read a pair ago
   };
