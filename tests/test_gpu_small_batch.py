@@ -87,3 +87,20 @@ def test_mul_mat_id_pairs(hip, fmt, ne11):
     _lib.launch_log()
     run_id(hip, fmt, 768, 50, 5, 2, ne11, 14, ids, pad_w=1 if fmt in ("mxfp4", "q6_k", "nvfp4") else 2)
     assert "small_mfma_gemm_grouped" in _lib.launch_log()
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("pad", [0, 1])
+def test_many_rows_no_gemm_takes(hip, fmt, pad):
+    """More rows than a small batch where the prefill GEMM does not take the
+    weights: rows off 4-byte alignment (pad), an odd superblock count (IQ2)."""
+    pad_w = 0 if not pad else 1 if fmt in ("mxfp4", "q6_k", "nvfp4") else 2
+    names = launched(hip, fmt, 768, 75, 70, pad_w=pad_w, pad_y=1)
+    if pad_w or fmt.startswith("iq2"):
+        assert "small_mfma_gemm" in names, names
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q4_1", "mxfp4", "nvfp4"])
+def test_many_quantized_rows(hip, fmt):
+    # a Q8_0 / Q8_1 src1, which those formats' GEMMs do not read
+    assert launched(hip, fmt, 512, 75, 70, prequant=True) == ["small_mfma_gemm"]

@@ -215,15 +215,17 @@ void mul_mat_id_kq_grouped(bool q6, const uint8_t* W, const uint8_t* Xq, float* 
                            const RowStrides& st, const PairArgs& pr, int n_pairs, void* ws);
 
 // Small-batch mul_mat (small_batch.hip): 2 .. kSmallBatchRows activation rows
-// on one 16-row-wide MFMA GEMM whose waves split K, any format (decode_quantized's
-// codes, Q4_K = 8), record alignment and K.  X is quantized into Xq; _quantized
-// reads Xq.  False, with nothing launched, when the call does not suit it.
+// on one 16-row-wide MFMA GEMM whose waves split K, any format
+// (decode_quantized's codes, Q4_K = 8) and record alignment, K of whole
+// 256-value units.  X is quantized into Xq; _quantized reads Xq.  gemm: the
+// format's prefill GEMM takes the call too, so the faster one runs; without
+// one it takes any number of rows.  False, with nothing launched, when the
+// call does not suit it.
 constexpr size_t kSmallBatchRows = 64;
 bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* tab0, const void* tab1,
-                 float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
+                 float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm = true);
 bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
-                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
-
+                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm = true);
 // MUL_MAT_ID's (token, slot) pairs on the same kernel, 2 .. 64 of them, which
 // groups them by expert itself: Xq holds the x_rows quantized src1 rows
 // (token * ne11 + row).  _ok: whether the shape suits it.

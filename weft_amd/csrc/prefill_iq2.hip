@@ -490,8 +490,11 @@ void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t
                      const int8_t* signs, float* Y, size_t N, size_t K, size_t M,
                      const RowStrides& st) {
   if (small_batch(2, W, X, Xq, grid, signs, Y, N, K, M, st)) return;
-  if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok(W, Xq, Y, grid, signs, N, K, M, st))
-    return decode_iq2_xxs(W, X, Xq, grid, signs, Y, N, K, M, st);
+  if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok(W, Xq, Y, grid, signs, N, K, M, st)) {
+    if (!small_batch(2, W, X, Xq, grid, signs, Y, N, K, M, st, false))
+      decode_iq2_xxs(W, X, Xq, grid, signs, Y, N, K, M, st);
+    return;
+  }
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);
   gemm_iq2(W, Xq, grid, signs, Y, N, K, M, st);
 }
@@ -500,8 +503,11 @@ void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t
 void mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid, const int8_t* signs,
                     float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
   if (small_batch(7, W, X, Xq, grid, signs, Y, N, K, M, st)) return;
-  if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok<true>(W, Xq, Y, grid, signs, N, K, M, st))
-    return decode_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, st);
+  if (X == nullptr || !aligned(X, 4) || !gemm_iq2_ok<true>(W, Xq, Y, grid, signs, N, K, M, st)) {
+    if (!small_batch(7, W, X, Xq, grid, signs, Y, N, K, M, st, false))
+      decode_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, st);
+    return;
+  }
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);
   gemm_iq2<true>(W, Xq, grid, signs, Y, N, K, M, st);
 }

@@ -467,8 +467,11 @@ void gemm_kq(const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K, 
 void mul_mat_q6k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
                  const RowStrides& st) {
   if (small_batch(3, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
-  if (X == nullptr || !aligned(X, 4) || !gemm_kq_ok<KQ::Q6_K>(W, Xq, Y, N, K, M, st))
-    return decode_q6_k(W, X, Xq, Y, N, K, M, st);
+  if (X == nullptr || !aligned(X, 4) || !gemm_kq_ok<KQ::Q6_K>(W, Xq, Y, N, K, M, st)) {
+    if (!small_batch(3, W, X, Xq, nullptr, nullptr, Y, N, K, M, st, false))
+      decode_q6_k(W, X, Xq, Y, N, K, M, st);
+    return;
+  }
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);
   gemm_kq<KQ::Q6_K>(W, Xq, Y, N, K, M, st);
 }
@@ -491,8 +494,11 @@ bool gemm_kq_try(bool q6, const uint8_t* W, const float* X, uint8_t* Xq, float* 
 void mul_mat_q5k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
                  const RowStrides& st) {
   if (small_batch(4, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
-  if (X == nullptr || !aligned(X, 4) || !gemm_kq_ok<KQ::Q5_K>(W, Xq, Y, N, K, M, st))
-    return decode_q5_k(W, X, Xq, Y, N, K, M, st);
+  if (X == nullptr || !aligned(X, 4) || !gemm_kq_ok<KQ::Q5_K>(W, Xq, Y, N, K, M, st)) {
+    if (!small_batch(4, W, X, Xq, nullptr, nullptr, Y, N, K, M, st, false))
+      decode_q5_k(W, X, Xq, Y, N, K, M, st);
+    return;
+  }
   quantize_q8_k_rows(X, st.ldx, Xq, M, K);
   gemm_kq<KQ::Q5_K>(W, Xq, Y, N, K, M, st);
 }

@@ -627,7 +627,7 @@ void mul_mat_q4k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t
       gemm_q4k_ok(W, N, K, M, st)) {
     quantize_q8_k_rows(X, st.ldx, Xq, M, K);
     gemm_q4k(W, Xq, Y, N, K, M, st);
-  } else {
+  } else if (!small_batch(8, W, X, Xq, nullptr, nullptr, Y, N, K, M, st, false)) {
     decode_q4k(W, X, Xq, Y, N, K, M, st);
   }
 }

@@ -1136,7 +1136,8 @@ void mul_mat_q4_0(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
   if (N == 0 || M == 0 || K == 0) return decode_q4_0(W, X, Xq, Y, N, K, M, st);
   if (small_batch(0, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
-      !prefill_q80<WFmt::Q4_0>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st))
+      (!prefill_q80<WFmt::Q4_0>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st) &&
+       !small_batch(0, W, X, Xq, nullptr, nullptr, Y, N, K, M, st, false)))
     decode_q4_0(W, X, Xq, Y, N, K, M, st);
 }
 
@@ -1145,7 +1146,8 @@ void mul_mat_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
   if (N == 0 || M == 0 || K == 0) return decode_q4_1(W, X, Xq, Y, N, K, M, st);
   if (small_batch(6, W, X, Xq, nullptr, nullptr, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
-      !prefill_q80<WFmt::Q4_1>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st))
+      (!prefill_q80<WFmt::Q4_1>(W, X, Xq, nullptr, nullptr, Y, N, K, M, st) &&
+       !small_batch(6, W, X, Xq, nullptr, nullptr, Y, N, K, M, st, false)))
     decode_q4_1(W, X, Xq, Y, N, K, M, st);
 }
 
@@ -1154,7 +1156,8 @@ void mul_mat_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* 
   if (N == 0 || M == 0 || K == 0) return decode_nvfp4(W, X, Xq, codebook, ue4m3, Y, N, K, M, st);
   if (small_batch(5, W, X, Xq, codebook, ue4m3, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
-      !prefill_q80<WFmt::NVFP4>(W, X, Xq, codebook, ue4m3, Y, N, K, M, st))
+      (!prefill_q80<WFmt::NVFP4>(W, X, Xq, codebook, ue4m3, Y, N, K, M, st) &&
+       !small_batch(5, W, X, Xq, codebook, ue4m3, Y, N, K, M, st, false)))
     decode_nvfp4(W, X, Xq, codebook, ue4m3, Y, N, K, M, st);
 }
 
@@ -1163,7 +1166,8 @@ void mul_mat_mxfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* 
   if (N == 0 || M == 0 || K == 0) return decode_mxfp4(W, X, Xq, codebook, scale, Y, N, K, M, st);
   if (small_batch(1, W, X, Xq, codebook, scale, Y, N, K, M, st)) return;
   if (W == nullptr || X == nullptr || Xq == nullptr || Y == nullptr ||
-      !prefill_q80<WFmt::MXFP4>(W, X, Xq, codebook, scale, Y, N, K, M, st))
+      (!prefill_q80<WFmt::MXFP4>(W, X, Xq, codebook, scale, Y, N, K, M, st) &&
+       !small_batch(1, W, X, Xq, codebook, scale, Y, N, K, M, st, false)))
     decode_mxfp4(W, X, Xq, codebook, scale, Y, N, K, M, st);
 }
 

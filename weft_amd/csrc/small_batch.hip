@@ -814,6 +814,7 @@ static bool small_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t*
   const TileBindings& tb = tile_bindings();
   return N > 0 && K > 0 && K % 256 == 0 && tb.nc == 0 && tb.mr == 0 && tb.mc == 0 && W != nullptr &&
          Xq != nullptr && Y != nullptr && N <= (size_t)INT32_MAX - 256 && K <= (size_t)INT32_MAX &&
+         M < ((size_t)1 << 24) && (M + 15) / 16 * ((N + 127) / 128) < ((size_t)1 << 27) &&
          M * f.x_row(K) < ((size_t)1 << 32) && std::max(st.ldw, K / f.elems * f.rec) < kMaxRow &&
          f.x_row(K) < kMaxRow && aligned(W, f.w_align) && aligned(Xq, f.x_align) && aligned(Y, 4) &&
          tables_ok(fmt, tab0, tab1) && strides_ok(st, K / f.elems * f.rec, f.w_align, K, N, N, 1);
@@ -830,11 +831,12 @@ static bool small_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t*
 // both grow with K.  The limits are where the two lines measured at 4096 and
 // 11008 x 4096, 16 .. 64 rows, cross (MXFP4, 64 rows: 20.7 against 33.0 us
 // at 4096 rows, 41.0 against 35.3 at 11008).
-static bool small_wins(int fmt, size_t N, size_t M) {
+static bool small_wins(int fmt, size_t N, size_t M, bool gemm) {
   static constexpr uint8_t kFrom[9] = {3, 4, 3, 4, 2, 4, 3, 4, 2};
-  static constexpr uint16_t kLimit[9] = {21000, 14000, 20000, 25000, 27000, 28000, 21000, 28000, 8192};
-  if (M < kFrom[fmt] || M > kSmallBatchRows) return false;
-  if (M < 16) return true;
+  static constexpr uint16_t kLimit[9] = {21000, 14000, 20000, 17000, 27000, 28000, 21000, 18000, 8192};
+  if (M < kFrom[fmt]) return false;
+  if (M < 16 || !gemm) return true;
+  if (M > kSmallBatchRows) return false;
   // one token tile of 16 costs five eighths of one of 32; Q4_K's GEMM is 1.5
   // times longer past 32 rows
   const size_t w = M <= 16 ? N * 5 / 8 : N * ((M + 31) / 32);
@@ -842,8 +844,8 @@ static bool small_wins(int fmt, size_t N, size_t M) {
 }
 
 bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
-                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
-  if (!small_wins(fmt, N, M) || st.ldy < N || st.ldy >= ((size_t)1 << 38) ||
+                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm) {
+  if (!small_wins(fmt, N, M, gemm) || st.ldy < N || st.ldy >= ((size_t)1 << 38) ||
       !small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, M, st)) return false;
   const FmtInfo f = fmt_info(fmt);
   const Args a{W, Xq, tab0, tab1, Y, (int)N, (int)K, (int)M, 1, (uint32_t)(N > 1 ? st.ldw : K / f.elems * f.rec),
@@ -867,8 +869,8 @@ void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab
 }
 
 bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* tab0, const void* tab1,
-                 float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
-  if (X == nullptr || !aligned(X, 4) || !small_wins(fmt, N, M) || st.ldx < K || st.ldy < N ||
+                 float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm) {
+  if (X == nullptr || !aligned(X, 4) || !small_wins(fmt, N, M, gemm) || st.ldx < K || st.ldy < N ||
       st.ldx >= ((size_t)1 << 38) || st.ldy >= ((size_t)1 << 38) || !small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, M, st))
     return false;
   switch (fmt) {
@@ -878,7 +880,7 @@ bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const i
     case 6: quantize_q8_1_rows(X, st.ldx, Xq, M, K); break;
     default: quantize_q8_k_rows(X, st.ldx, Xq, M, K); break;
   }
-  return small_batch_quantized(fmt, W, Xq, tab0, tab1, Y, N, K, M, st);
+  return small_batch_quantized(fmt, W, Xq, tab0, tab1, Y, N, K, M, st, gemm);
 }
 
 }  // namespace weft
