@@ -256,6 +256,20 @@ __device__ inline void stage_q8k_load(const uint8_t* __restrict__ xq, int K, int
   }
 }
 
+// The end of a batch-1 GEMV whose rows are split into KS steps over KS waves:
+// rows [row_base, row_end) are their steps' partial sums (part[row - row_base]
+// [step]) added in step order.  Every thread of the workgroup calls it.
+template <int KS>
+__device__ __forceinline__ void gemv_add_steps(const float* part, float* Y, int row_base, int row_end) {
+  __syncthreads();
+  for (int r = threadIdx.x; r < row_end - row_base; r += blockDim.x) {
+    float y = part[r * KS];
+#pragma unroll
+    for (int s = 1; s < KS; ++s) y += part[r * KS + s];
+    Y[row_base + r] = y;
+  }
+}
+
 // ---------------------------------------------------------------- Q8_0
 // LDS image of one Q8_0 activation row: int8 qs[K] | float d[K/32]
 // (d is the fp16 scale widened to fp32, as the vec_dot reads it).

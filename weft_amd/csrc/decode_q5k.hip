@@ -1,6 +1,6 @@
 // Batch-1 decode GEMV for Q5_K x Q8_K: production_mul_mat_q5_k_decode /
 // production_mul_mat_q5_k at M = 1 (examples/kernels/mul_mat/q5_k_decode.py,
-// q5_k.py:9-37), rows of up to 4096 values.
+// q5_k.py:9-37), rows of up to 4 * 4096 values.
 //
 // Semantics (ggml_vec_dot_q5_K_q8_K_generic, ggml-cpu/quants.c:720-798):
 //   y = sum_b dx_b * (dw_b * S_b - dmin_b * Mn_b)
@@ -42,19 +42,30 @@ struct Q5Args {
   size_t ldw;
 };
 
+// Rows longer than one step of 4096 values (KS > 1): the waves form groups of
+// KS, wave w takes step w % KS (an even share of the superblocks, so its
+// activation slice still fits the registers) of the rows of group w / KS, and
+// the KS partial sums of a row are added in step order at the end.  One call,
+// against the staged GEMV: 4096 x 11008 13.8 -> 9.9 us, 14336 x 5120 20.3 ->
+// 14.3, 2000 x 14336 12.9 -> 8.0.
+template <int KS>
 __global__ void __launch_bounds__(kThreads) q5k_gemv_m1_kernel(Q5Args a) {
-  extern __shared__ __align__(16) char lds[];  // Q8_K activation row
+  constexpr int kGroups = kWaves / KS;
+  extern __shared__ __align__(16) char lds[];  // Q8_K activation row, then the steps' partial sums
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int K = a.K;
-  const int nsb = K >> 8;  // <= 16
-  const bool live = lane < 4 * nsb;
-  const int sb = min(lane >> 2, nsb - 1), g = lane & 3;
+  const int nsb = K >> 8;  // <= 16 KS
+  const int st = wave % KS, grp = wave / KS;
+  const int spb = (nsb + KS - 1) / KS;  // <= 16
+  const bool live = (lane >> 2) < spb && st * spb + (lane >> 2) < nsb;
+  const int sb = min(st * spb + (lane >> 2), nsb - 1), g = lane & 3;
+  float* part = reinterpret_cast<float*>(lds + q8k_lds_row_bytes(K));  // [row - row_base][step]
   const uint32_t off = (uint32_t)(kQ5_KBytes * sb);  // 16-byte aligned
   const size_t rb = a.ldw;
-  const int row_first = blockIdx.x * a.rows_per_wg + wave;
-  const int row_end = min(a.N, blockIdx.x * a.rows_per_wg + a.rows_per_wg);
-  const int nrows = row_first < row_end ? (row_end - row_first + kWaves - 1) / kWaves : 0;
+  const int row_base = blockIdx.x * a.rows_per_wg, row_first = row_base + grp;
+  const int row_end = min(a.N, row_base + a.rows_per_wg);
+  const int nrows = grp < kGroups && row_first < row_end ? (row_end - row_first + kGroups - 1) / kGroups : 0;
 
   // activation loads first: waiting for them does not wait for the weights
   Q8KStager16<1> stager;
@@ -65,7 +76,7 @@ __global__ void __launch_bounds__(kThreads) q5k_gemv_m1_kernel(Q5Args a) {
     uint4 h, qh0, qh1, q0, q1;
   };
   auto issue = [&](RowBuf& buf, int k) {
-    const int row = min(row_first + k * kWaves, a.N - 1);  // clamped: always a valid row
+    const int row = min(row_first + k * kGroups, a.N - 1);  // clamped: always a valid row
     const uint8_t* rec = a.W + (size_t)row * rb + off;
     buf.h = *reinterpret_cast<const uint4*>(rec);
     buf.qh0 = *reinterpret_cast<const uint4*>(rec + 16);
@@ -123,7 +134,12 @@ __global__ void __launch_bounds__(kThreads) q5k_gemv_m1_kernel(Q5Args a) {
     const float t = dx * (dw * (float)S - dmin * (float)Mn);
     // lanes past the row's last superblock duplicate it: they add exactly 0
     const float tot = wave_sum_f(live ? t : 0.f);
-    if (lane == 0) a.Y[row_first + k * kWaves] = tot;
+    if (lane == 0) {
+      if constexpr (KS == 1)
+        a.Y[row_first + k * kGroups] = tot;
+      else
+        part[(row_first + k * kGroups - row_base) * KS + st] = tot;
+    }
   };
 
   int k = 0;
@@ -140,25 +156,28 @@ __global__ void __launch_bounds__(kThreads) q5k_gemv_m1_kernel(Q5Args a) {
   } else if (nrows - k == 1) {
     compute(bufA, k);
   }
+  if constexpr (KS > 1) gemv_add_steps<KS>(part, a.Y, row_base, row_end);
 }
 
 }  // namespace
 
 // Launches the kernel above when the call suits it: one activation row of
-// K <= 4096, 16-byte aligned X and W with rows a multiple of 16 bytes apart,
+// K <= 4 * 4096, 16-byte aligned X and W with rows a multiple of 16 bytes apart,
 // Xq 4-byte aligned.
 bool decode_q5k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st) {
   const size_t rb = K / 256 * kQ5_KBytes;
   const size_t ldw = N > 1 ? st.ldw : rb;
-  if (N == 0 || K == 0 || K > 4096 || K % 256 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
+  if (N == 0 || K == 0 || K > 4 * 4096 || K % 256 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
       Y == nullptr || !aligned(X, 16) || !aligned(W, 16) || ldw % 16 != 0 || !aligned(Y, 4) ||
       !aligned(Xq, 4) || N > (size_t)INT32_MAX || (N > 1 && ldw < rb) || ldw >= ((size_t)1 << 40))
     return false;
   // one workgroup per CU (79 VGPRs: a second one would not be resident;
   // measured 8.7 us for two per CU against 7.95 us at 11008 x 4096)
   const int cus = cu_count();
-  const size_t wgs = std::max<size_t>(1, std::min<size_t>((size_t)cus, (N + kWaves - 1) / kWaves));
+  const int ks = (int)((K + 4095) / 4096);
+  const size_t groups = (size_t)(kWaves / ks);  // rows a workgroup works on at once
+  const size_t wgs = std::max<size_t>(1, std::min<size_t>((size_t)cus, (N + groups - 1) / groups));
   Q5Args a;
   a.W = W;
   a.X = X;
@@ -171,7 +190,14 @@ bool decode_q5k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size
   a.rows_per_wg = nc > 0 ? (int)std::min<size_t>(N, (size_t)nc) : (int)((N + wgs - 1) / wgs);
   a.ldw = ldw;
   const int grid = (int)((N + a.rows_per_wg - 1) / a.rows_per_wg);
-  q5k_gemv_m1_kernel<<<grid, kThreads, q8k_lds_row_bytes((int)K), current_stream()>>>(a);
+  const size_t lds = q8k_lds_row_bytes((int)K) + (ks > 1 ? 4 * (size_t)ks * a.rows_per_wg : 0);
+  if (lds > max_lds_per_block()) return false;
+  switch (ks) {
+    case 1: q5k_gemv_m1_kernel<1><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 2: q5k_gemv_m1_kernel<2><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 3: q5k_gemv_m1_kernel<3><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    default: q5k_gemv_m1_kernel<4><<<grid, kThreads, lds, current_stream()>>>(a); break;
+  }
   check_launch("q5k_gemv_m1_kernel");
   return true;
 }

@@ -1,6 +1,6 @@
 // Batch-1 decode GEMV for Q6_K x Q8_K: production_mul_mat_q6_k_decode /
 // production_mul_mat_q6_k at M = 1 (examples/kernels/mul_mat/q6_k_decode.py,
-// q6_k.py:9-37), rows of up to 4096 values.
+// q6_k.py:9-37), rows of up to 4 * 4096 values.
 //
 // Semantics (ggml_vec_dot_q6_K_q8_K_generic, ggml-cpu/quants.c:800-853):
 //   y = sum_b (dw_b dx_b) * sum_{j<16} sc_j * sum_{16} (q6 - 32) * x      (exact int32)
@@ -42,25 +42,43 @@ struct Q6Args {
   size_t ldw;
 };
 
+// Rows longer than one step of 4096 values (KS > 1): the waves form groups of
+// KS, wave w takes step w % KS (an even share of the superblocks, so its
+// activation slice still fits the registers) of the rows of group w / KS, and
+// the KS partial sums of a row are added in step order at the end.
+// One call, against the staged GEMV, whose rows all pass through LDS: 4096 x
+// 11008 (43 superblocks, 2-byte rows) 14.6 -> 13.1 us, 14336 x 5120 22.1 ->
+// 18.2, 2000 x 14336 13.2 -> 9.7.
+// kOdd: rows that are only 2-byte aligned, so a lane's shift is its row's.
+template <int KS, bool kOdd>
 __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
-  extern __shared__ __align__(16) char lds[];  // Q8_K activation row
+  constexpr int kGroups = kWaves / KS;
+  extern __shared__ __align__(16) char lds[];  // Q8_K activation row, then the steps' partial sums
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int K = a.K;
-  const int nsb = K >> 8;  // <= 16
-  const bool live = lane < 4 * nsb;
-  const int sb = min(lane >> 2, nsb - 1), g = lane & 3, h = g >> 1;
+  const int nsb = K >> 8;  // <= 16 KS
+  const int st = wave % KS, grp = wave / KS;
+  const int spb = (nsb + KS - 1) / KS;  // <= 16
+  const bool live = (lane >> 2) < spb && st * spb + (lane >> 2) < nsb;
+  const int sb = min(st * spb + (lane >> 2), nsb - 1), g = lane & 3, h = g >> 1;
+  float* part = reinterpret_cast<float*>(lds + q8k_lds_row_bytes(K));  // [row - row_base][step]
   const uint32_t rec = (uint32_t)(kQ6_KBytes * sb);
-  const uint32_t sh = rec & 3u;   // 0 or 2
-  const uint32_t base = rec - sh;  // dword holding the record's first byte
-  // the lane's regions, relative to base: ql [sh + 64h, +64), qh
+  // offset of the record from the dword holding its first byte (0 or 2); kOdd:
+  // row by row
+  const uint32_t sh_even = rec & 3u;
+  auto shift = [&](int row) -> uint32_t {
+    if constexpr (!kOdd) return sh_even;
+    return ((uint32_t)(uintptr_t)a.W + (uint32_t)row * (uint32_t)a.ldw + rec) & 2u;
+  };
+  // the lane's regions, from the record's offset - sh on: ql [sh + 64h, +64), qh
   // [sh + 128 + 32h, +32), scales [sh + 192 + 4g, +4), d [sh + 208, +2)
-  const uint32_t o_ql = base + 64 * h, o_qh = base + 128 + 32 * h, o_sc = base + 192 + 4 * g;
-  const uint32_t o_d = base + 208;
+  const uint32_t o_ql = rec + 64 * h, o_qh = rec + 128 + 32 * h, o_sc = rec + 192 + 4 * g;
+  const uint32_t o_d = rec + 208;
   const size_t rb = a.ldw;
-  const int row_first = blockIdx.x * a.rows_per_wg + wave;
-  const int row_end = min(a.N, blockIdx.x * a.rows_per_wg + a.rows_per_wg);
-  const int nrows = row_first < row_end ? (row_end - row_first + kWaves - 1) / kWaves : 0;
+  const int row_base = blockIdx.x * a.rows_per_wg, row_first = row_base + grp;
+  const int row_end = min(a.N, row_base + a.rows_per_wg);
+  const int nrows = grp < kGroups && row_first < row_end ? (row_end - row_first + kGroups - 1) / kGroups : 0;
 
   Q8KStager16<1> stager;
   stager.prefetch(a.X, (size_t)K, K, 0, 1);
@@ -73,8 +91,9 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
     uint32_t ql[17], qh[9], sc[2], d;
   };
   auto issue = [&](RowBuf& buf, int k) {
-    const int row = min(row_first + k * kWaves, a.N - 1);  // clamped: always a valid row
-    const uint8_t* rp = a.W + (size_t)row * rb;
+    const int row = min(row_first + k * kGroups, a.N - 1);  // clamped: always a valid row
+    const uint32_t sh = shift(row);
+    const uint8_t* rp = a.W + (size_t)row * rb - sh;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(rp + o_ql + 16 * i);
@@ -127,6 +146,7 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   const uint32_t hsh = 4 * (g & 1);        // qh bit pairs 2s: s = 2 (g & 1) and 2 (g & 1) + 1
 
   auto compute = [&](const RowBuf& buf, int k) {
+    const uint32_t sh = shift(row_first + k * kGroups);
     uint32_t ql[16], qh[8];
 #pragma unroll
     for (int i = 0; i < 16; ++i) ql[i] = __builtin_amdgcn_alignbyte(buf.ql[i + 1], buf.ql[i], sh);  // sh 0 or 2
@@ -154,7 +174,12 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
     const int bsum = sum4(live ? tot : 0);  // the superblock's four lanes
     const float t = (lane & 3) == 0 && live ? (dw * dx) * (float)bsum : 0.f;
     const float y = wave_sum_f(t);
-    if (lane == 0) a.Y[row_first + k * kWaves] = y;
+    if (lane == 0) {
+      if constexpr (KS == 1)
+        a.Y[row_first + k * kGroups] = y;
+      else
+        part[(row_first + k * kGroups - row_base) * KS + st] = y;
+    }
   };
 
   int k = 0;
@@ -171,24 +196,38 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   } else if (nrows - k == 1) {
     compute(bufA, k);
   }
+  if constexpr (KS > 1) gemv_add_steps<KS>(part, a.Y, row_base, row_end);
 }
 
 }  // namespace
 
+namespace {
+template <bool kOdd>
+void launch_steps(int ks, int grid, size_t lds, const Q6Args& a) {
+  switch (ks) {
+    case 1: q6k_gemv_m1_kernel<1, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 2: q6k_gemv_m1_kernel<2, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 3: q6k_gemv_m1_kernel<3, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    default: q6k_gemv_m1_kernel<4, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
+  }
+}
+}  // namespace
+
 // Launches the kernel above when the call suits it: one activation row of
-// K <= 4096 with an even superblock count (4-byte aligned rows), 16-byte
-// aligned X, W 4-byte aligned with rows a multiple of 4 bytes apart, Xq
-// 4-byte aligned.
+// K <= 4 * 4096, 16-byte aligned X, W 2-byte aligned with rows a multiple of 2
+// bytes apart, Xq 4-byte aligned.
 bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st) {
   const size_t rb = K / 256 * kQ6_KBytes;
   const size_t ldw = N > 1 ? st.ldw : rb;
-  if (N == 0 || K == 0 || K > 4096 || K % 512 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
-      Y == nullptr || !aligned(X, 16) || !aligned(W, 4) || ldw % 4 != 0 || !aligned(Y, 4) ||
+  if (N == 0 || K == 0 || K > 4 * 4096 || K % 256 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
+      Y == nullptr || !aligned(X, 16) || !aligned(W, 2) || ldw % 2 != 0 || !aligned(Y, 4) ||
       !aligned(Xq, 4) || N > (size_t)INT32_MAX || (N > 1 && ldw < rb) || ldw >= ((size_t)1 << 40))
     return false;
   const int cus = cu_count();
-  const size_t wgs = std::max<size_t>(1, std::min<size_t>((size_t)cus, (N + kWaves - 1) / kWaves));
+  const int ks = (int)((K + 4095) / 4096);
+  const size_t groups = (size_t)(kWaves / ks);  // rows a workgroup works on at once
+  const size_t wgs = std::max<size_t>(1, std::min<size_t>((size_t)cus, (N + groups - 1) / groups));
   Q6Args a;
   a.W = W;
   a.X = X;
@@ -201,7 +240,12 @@ bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size
   a.rows_per_wg = nc > 0 ? (int)std::min<size_t>(N, (size_t)nc) : (int)((N + wgs - 1) / wgs);
   a.ldw = ldw;
   const int grid = (int)((N + a.rows_per_wg - 1) / a.rows_per_wg);
-  q6k_gemv_m1_kernel<<<grid, kThreads, q8k_lds_row_bytes((int)K), current_stream()>>>(a);
+  const size_t lds = q8k_lds_row_bytes((int)K) + (ks > 1 ? 4 * (size_t)ks * a.rows_per_wg : 0);
+  if (lds > max_lds_per_block()) return false;
+  if (K % 512 != 0 || !aligned(W, 4) || ldw % 4 != 0)
+    launch_steps<true>(ks, grid, lds, a);
+  else
+    launch_steps<false>(ks, grid, lds, a);
   check_launch("q6k_gemv_m1_kernel");
   return true;
 }

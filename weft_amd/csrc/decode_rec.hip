@@ -3,7 +3,7 @@
 // (36 bytes per 64 values): production_mul_mat_{q4_0,mxfp4,q4_1,nvfp4}_decode
 // at M = 1 (examples/kernels/mul_mat/q4_0_decode.py:10-20,
 // mxfp4_decode.py:10-23, q4_1_decode.py:10-11, nvfp4_decode.py), rows of up
-// to 4096 values.
+// to 4 * 4096 values.
 //
 // Semantics (GGML generic vec_dots, ggml-cpu/quants.c):
 //   Q4_0  :174-208  y = sum_b (I_b * dw_b) * dx_b,   I_b = sum_32 (q - 8) * x
@@ -62,8 +62,15 @@ __device__ __forceinline__ int rec_lookup16(uint32_t n, uint32_t c0, uint32_t c1
 
 enum class RF { Q4_0, MXFP4, Q4_1, NVFP4 };
 
-template <RF F>
+// Rows longer than one step of 4096 values (KS > 1): the waves form groups of
+// KS, wave w takes step w % KS (an even share of the lanes' 64 values, so its
+// activation slice still fits the registers) of the rows of group w / KS, and
+// the KS partial sums of a row are added in step order at the end.  One call,
+// against the staged GEMV: Q4_0 4096 x 11008 13.4 -> 9.0 us, 14336 x 5120 15.0
+// -> 11.3, MXFP4 15.2 -> 12.0 and 18.1 -> 17.2, NVFP4 14.6 -> 10.0.
+template <RF F, int KS>
 __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
+  constexpr int kGroups = kRecWaves / KS;
   constexpr bool kMx = F == RF::MXFP4;
   constexpr bool kNv = F == RF::NVFP4;
   constexpr bool kQ1 = F == RF::Q4_1;
@@ -77,10 +84,14 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int K = a.K;
-  const int nrec = K >> 5;     // 32-value blocks: even, <= 128
+  const int nrec = K >> 5;     // 32-value blocks: even, <= 128 KS
   const int nlanes = nrec >> 1;
-  const bool live = lane < nlanes;
-  const int j = min(lane, nlanes - 1);
+  const int st = wave % KS, grp = wave / KS;
+  const int lpb = (nlanes + KS - 1) / KS;  // lanes of a step, <= 64
+  const bool live = lane < lpb && st * lpb + lane < nlanes;
+  const int j = min(st * lpb + lane, nlanes - 1);
+  // partial sums [row - row_base][step], after the activation row
+  float* part = reinterpret_cast<float*>(act + (kQ1 ? q81_lds_row_bytes(K) : q80_lds_row_bytes(K)));
   const uint32_t boff = (uint32_t)(2 * kB * j);  // the lane's first byte in its row
   const uint32_t a0 = boff & ~3u, sh = boff & 3u;  // sh = 0 but for MXFP4 (0 or 2)
   const uint32_t row_bytes = (uint32_t)(nrec * kB);
@@ -88,23 +99,27 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
   // two bytes past them, which the row's last lane may not read
   const bool short9 = a0 + 36 > row_bytes;
   const size_t rb = a.ldw;
-  const int row_first = blockIdx.x * a.rows_per_wg + wave;
-  const int row_end = min(a.N, blockIdx.x * a.rows_per_wg + a.rows_per_wg);
-  const int nrows = row_first < row_end ? (row_end - row_first + kRecWaves - 1) / kRecWaves : 0;
+  const int row_base = blockIdx.x * a.rows_per_wg, row_first = row_base + grp;
+  const int row_end = min(a.N, row_base + a.rows_per_wg);
+  const int nrows = grp < kGroups && row_first < row_end ? (row_end - row_first + kGroups - 1) / kGroups : 0;
 
   // activation loads first (8 lanes per Q8_0 block, one 8-block step per
   // wave): waiting for them does not wait for the weight loads issued next
   const int nb = nrec;
-  const int b_act = 8 * wave + (lane >> 3);
-  float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (b_act < nb) xv = *reinterpret_cast<const float4*>(a.X + 32 * b_act + 4 * (lane & 7));
+  float4 xv[KS];
+#pragma unroll
+  for (int p = 0; p < KS; ++p) {
+    const int b = 8 * (wave + kRecWaves * p) + (lane >> 3);
+    xv[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (b < nb) xv[p] = *reinterpret_cast<const float4*>(a.X + 32 * b + 4 * (lane & 7));
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   struct RowBuf {
     uint32_t w[kW];
   };
   auto issue = [&](RowBuf& buf, int k) {
-    const int row = min(row_first + k * kRecWaves, a.N - 1);  // clamped: always a valid row
+    const int row = min(row_first + k * kGroups, a.N - 1);  // clamped: always a valid row
     const uint8_t* p = a.W + (size_t)row * rb + a0;
     const uint4 v0 = *reinterpret_cast<const uint4*>(p);
     const uint4 v1 = *reinterpret_cast<const uint4*>(p + 16);
@@ -132,8 +147,10 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
 
   if constexpr (kTab)
     if (threadIdx.x < 256) tab[threadIdx.x] = tsc;
-  {
-    const Q8_0Lane r = q80_quantize_8lanes(xv);
+#pragma unroll
+  for (int p = 0; p < KS; ++p) {
+    const int b_act = 8 * (wave + kRecWaves * p) + (lane >> 3);
+    const Q8_0Lane r = q80_quantize_8lanes(xv[p]);
     uint32_t sh16 = 0;
     if constexpr (kQ1) sh16 = q81_sum_half(r);  // every lane: a shuffle inside
     if (b_act < nb) {
@@ -198,6 +215,13 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
     c3 = ld_u32_a1(cb + 12);
   }
 
+  auto store = [&](float tot, int k) {
+    if (lane != 0) return;
+    if constexpr (KS == 1)
+      a.Y[row_first + k * kGroups] = tot;
+    else
+      part[(row_first + k * kGroups - row_base) * KS + st] = tot;
+  };
   auto compute = [&](const RowBuf& buf, int k) {
     const uint32_t* w = buf.w;
     float acc = 0.f;
@@ -215,8 +239,7 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
         I = dot4(rec_lookup16((u1 >> 4) & 0x0f0f0f0fu, c0, c1, c2, c3), x.w, I);
         acc += (dx[s >> 1] * tab[(w[0] >> (8 * s)) & 0xffu]) * (float)I;
       }
-      const float tot = wave_sum_f(live ? acc : 0.f);
-      if (lane == 0) a.Y[row_first + k * kRecWaves] = tot;
+      store(wave_sum_f(live ? acc : 0.f), k);
       return;
     }
 #pragma unroll
@@ -277,8 +300,7 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
         acc += (float)I * ws * dx[r];
     }
     // lanes past the row's last record duplicate it: they add exactly 0
-    const float tot = wave_sum_f(live ? acc : 0.f);
-    if (lane == 0) a.Y[row_first + k * kRecWaves] = tot;
+    store(wave_sum_f(live ? acc : 0.f), k);
   };
 
   // Issues inside the loop are unconditional so the in-order wait counts stay
@@ -297,12 +319,25 @@ __global__ void __launch_bounds__(kRecThreads) rec_gemv_m1_kernel(RecArgs a) {
   } else if (nrows - k == 1) {
     compute(bufA, k);
   }
+  if constexpr (KS > 1) gemv_add_steps<KS>(part, a.Y, row_base, row_end);
 }
 
 }  // namespace
 
+namespace {
+template <RF F>
+void launch_steps(int ks, int grid, size_t lds, const RecArgs& a) {
+  switch (ks) {
+    case 1: rec_gemv_m1_kernel<F, 1><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
+    case 2: rec_gemv_m1_kernel<F, 2><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
+    case 3: rec_gemv_m1_kernel<F, 3><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
+    default: rec_gemv_m1_kernel<F, 4><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
+  }
+}
+}  // namespace
+
 // Launches the kernel above when the call suits it: one activation row of
-// K <= 4096 (K a multiple of 64), 16-byte aligned X, weight rows at 4-byte
+// K <= 4 * 4096 (K a multiple of 64), 16-byte aligned X, weight rows at 4-byte
 // aligned addresses, the MXFP4 / NVFP4 scale table 4-byte aligned.
 // fmt: Q4_0 0, MXFP4 1, NVFP4 5, Q4_1 6.
 bool decode_rec_m1(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
@@ -312,14 +347,17 @@ bool decode_rec_m1(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const
   if (fmt != 0 && fmt != 1 && fmt != 5 && fmt != 6) return false;
   const size_t rb = K / 32 * rec;
   const size_t ldw = N > 1 ? st.ldw : rb;
-  if (N == 0 || K == 0 || K > 4096 || K % 64 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
+  if (N == 0 || K == 0 || K > 4 * 4096 || K % 64 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
       Y == nullptr || !aligned(X, 16) || !aligned(W, 4) || ldw % 4 != 0 || !aligned(Y, 4) ||
       !aligned(Xq, 2) || N > (size_t)INT32_MAX || (N > 1 && ldw < rb) || ldw >= ((size_t)1 << 40) ||
       (mx && (codebook == nullptr || scale == nullptr || !aligned(scale, 4))))
     return false;
   const int cus = cu_count();
-  // 16 rows per workgroup at least (one per wave), two workgroups per CU at most
-  const size_t wgs = std::max<size_t>(1, std::min<size_t>(2 * (size_t)cus, (N + kRecWaves - 1) / kRecWaves));
+  // a row per wave (or group of waves) at least; two workgroups per CU at
+  // most, one where each quantizes more than 4096 values
+  const int ks = (int)((K + 4095) / 4096);
+  const size_t groups = (size_t)(kRecWaves / ks), most = (size_t)(ks > 1 ? cus : 2 * cus);
+  const size_t wgs = std::max<size_t>(1, std::min<size_t>(most, (N + groups - 1) / groups));
   RecArgs a;
   a.W = W;
   a.X = X;
@@ -334,12 +372,14 @@ bool decode_rec_m1(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const
   a.rows_per_wg = nc > 0 ? (int)std::min<size_t>(N, (size_t)nc) : (int)((N + wgs - 1) / wgs);
   a.ldw = ldw;
   const int grid = (int)((N + a.rows_per_wg - 1) / a.rows_per_wg);
-  const size_t lds = 1024 + (fmt == 6 ? q81_lds_row_bytes((int)K) : q80_lds_row_bytes((int)K));
+  const size_t lds = 1024 + (fmt == 6 ? q81_lds_row_bytes((int)K) : q80_lds_row_bytes((int)K)) +
+                     (ks > 1 ? 4 * (size_t)ks * a.rows_per_wg : 0);
+  if (lds > max_lds_per_block()) return false;
   switch (fmt) {
-    case 1: rec_gemv_m1_kernel<RF::MXFP4><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
-    case 5: rec_gemv_m1_kernel<RF::NVFP4><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
-    case 6: rec_gemv_m1_kernel<RF::Q4_1><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
-    default: rec_gemv_m1_kernel<RF::Q4_0><<<grid, kRecThreads, lds, current_stream()>>>(a); break;
+    case 1: launch_steps<RF::MXFP4>(ks, grid, lds, a); break;
+    case 5: launch_steps<RF::NVFP4>(ks, grid, lds, a); break;
+    case 6: launch_steps<RF::Q4_1>(ks, grid, lds, a); break;
+    default: launch_steps<RF::Q4_0>(ks, grid, lds, a); break;
   }
   check_launch("rec_gemv_m1_kernel");
   return true;

@@ -50,16 +50,16 @@ void decode_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* c
 
 // Batch-1 Q4_0 (fmt 0) / MXFP4 (1) / NVFP4 (5) / Q4_1 (6) GEMV with the records in VGPRs
 // (decode_rec.hip); false, with nothing launched, when the call does not
-// suit it (K > 4096, unaligned operands), for the caller's general kernel.
+// suit it (K > 4 * 4096, unaligned operands), for the caller's general kernel.
 bool decode_rec_m1(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                    const float* scale, float* Y, size_t N, size_t K, const RowStrides& st);
 // Batch-1 Q5_K GEMV with the records in VGPRs (decode_q5k.hip); false, with
-// nothing launched, when the call does not suit it (K > 4096, W or its rows
-// not 16-byte aligned).
+// nothing launched, when the call does not suit it (K > 4 * 4096, W or its
+// rows not 16-byte aligned).
 bool decode_q5k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st);
 // Batch-1 Q6_K GEMV with the records in VGPRs (decode_q6k.hip); false when
-// the call does not suit it (K > 4096, an odd superblock count, unaligned).
+// the call does not suit it (K > 4 * 4096, unaligned).
 bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st);
 // Batch-1 IQ2_XXS / IQ2_XS (xs) GEMV with the records in VGPRs (decode_iq2.hip);
