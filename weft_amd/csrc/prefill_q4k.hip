@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(TL::kThreads, 1) q4k_mfma_gemm(GemmArgs a) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   if (tid < 4) zero16[tid] = 0u;
-  // Tile t of the launch: m-tile fastest (dense) or expert tile fastest
+  // Tile t of the launch: banded (dense, tile_store.h) or expert tile fastest
   // (grouped: m0 then indexes the pair list, and the tiles are the device's
   // tile count, not the host's bound, so the schedule below spreads only real
   // tiles).  Every wave enumerates the same tiles.
@@ -212,12 +212,15 @@ __global__ void __launch_bounds__(TL::kThreads, 1) q4k_mfma_gemm(GemmArgs a) {
   auto tile_info = [&](int t, Tile& ti) -> bool {
     if constexpr (kGroup) {
       if (!group_tile(a.grp, t % ntm, ti.m0, ti.mrows, ti.w_off)) return false;
+      ti.n0 = (t / ntm) * kNT;
     } else {
-      ti.m0 = (t % ntm) * kMT;
+      int tm, tn;
+      banded_tile(t, ntm, ntn, tm, tn);
+      ti.m0 = tm * kMT;
+      ti.n0 = tn * kNT;
       ti.mrows = min(kMT, a.M - ti.m0);
       ti.w_off = 0;
     }
-    ti.n0 = (t / ntm) * kNT;
     ti.m0 = __builtin_amdgcn_readfirstlane(ti.m0);
     ti.mrows = __builtin_amdgcn_readfirstlane(ti.mrows);
     ti.n0 = __builtin_amdgcn_readfirstlane(ti.n0);

@@ -215,16 +215,19 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
   const uint8_t* W = a.W;
   {
     const int ntm = kGroup ? a.grp.tmax : (a.M + kMT - 1) / kMT;
-    const int Tn = ntm * ((a.N + kNT - 1) / kNT);
+    const int ntn = (a.N + kNT - 1) / kNT, Tn = ntm * ntn;
     const int L = blockIdx.x, x = L & 7, j = L >> 3;
     const int t = x * (Tn >> 3) + min(x, Tn & 7) + j;
-    n0 = (t / ntm) * kNT;
     if constexpr (kGroup) {
+      n0 = (t / ntm) * kNT;
       long long w_off;
       if (!group_tile(a.grp, t % ntm, m0, mrows, w_off)) return;  // no barrier yet
       W += w_off;
     } else {
-      m0 = (t % ntm) * kMT;
+      int tm, tn;
+      banded_tile(t, ntm, ntn, tm, tn);
+      m0 = tm * kMT;
+      n0 = tn * kNT;
       mrows = min(kMT, a.M - m0);
     }
   }
@@ -736,16 +739,19 @@ __device__ void scaled_body(const GemmArgs& a, uint8_t* lds) {
   const uint8_t* W = a.W;
   {
     const int ntm = kGroup ? a.grp.tmax : (a.M + kMT - 1) / kMT;
-    const int Tn = ntm * ((a.N + kNT - 1) / kNT);
+    const int ntn = (a.N + kNT - 1) / kNT, Tn = ntm * ntn;
     const int L = blockIdx.x, x = L & 7, j = L >> 3;
     const int t = x * (Tn >> 3) + min(x, Tn & 7) + j;
-    n0 = __builtin_amdgcn_readfirstlane((t / ntm) * kNT);
     if constexpr (kGroup) {
+      n0 = __builtin_amdgcn_readfirstlane((t / ntm) * kNT);
       long long w_off;
       if (!group_tile(a.grp, t % ntm, m0, mrows, w_off)) return;  // no barrier yet
       W += w_off;
     } else {
-      m0 = __builtin_amdgcn_readfirstlane((t % ntm) * kMT);
+      int tm, tn;
+      banded_tile(t, ntm, ntn, tm, tn);
+      m0 = __builtin_amdgcn_readfirstlane(tm * kMT);
+      n0 = __builtin_amdgcn_readfirstlane(tn * kNT);
       mrows = min(kMT, a.M - m0);
     }
   }
