@@ -171,6 +171,7 @@ constexpr int q80_lds_bytes() {
 template <WFmt F, bool kGroup>
 __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
   using T = WTraits<F>;
+  constexpr bool kFactor = F == WFmt::Q4_0 || F == WFmt::Q4_1;  // dx dw from an MFMA
   constexpr int kRB = 8 * T::kRec;           // raw weight bytes per row and stage
   constexpr int kRL = w_lds_row<F>();        // LDS bytes per weight row (Q4_1: kRB + 4)
   constexpr int kWT = kNT * kRL;             // 18432 (Q4_0) / 17408 (MXFP4) / 20992 (Q4_1)
@@ -191,6 +192,7 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
   uint8_t* ring0 = lds;
   uint8_t* ring1 = lds + 2 * kStage;
   float(*adt)[2][8 * kMT] = reinterpret_cast<float(*)[2][8 * kMT]>(lds + 4 * kStage);  // [slot][parity][block][token]
+  // (kFactor: 64 fp16 scales, then the 64 zeros the kg half's operand slots read, per block)
   // Q4_1: the tokens' fp16 block sums [slot][parity][block][token]; MXFP4: scale table
   // [slot][parity][token][block]
   uint16_t(*ast)[2][8 * kMT] = reinterpret_cast<uint16_t(*)[2][8 * kMT]>(lds + 4 * kStage + 2 * 2 * 8 * kMT * 4);
@@ -310,10 +312,16 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
     if constexpr (F == WFmt::Q4_1) sraw = *reinterpret_cast<const uint4*>(dsrc + a.K / 16 + 16 * (size_t)st);
   };
   auto store_dx = [&](int slot) {
-    float* d = &adt[slot][par][0];
     const uint32_t w[4] = {dxraw.x, dxraw.y, dxraw.z, dxraw.w};
+    if constexpr (kFactor) {  // as they are, for the factor MFMA's operand
+      uint16_t* d = reinterpret_cast<uint16_t*>(&adt[slot][par][0]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) d[j * kMT + lane] = fp16_to_fp32((w[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+      for (int j = 0; j < 8; ++j) d[2 * j * kMT + lane] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+    } else {
+      float* d = &adt[slot][par][0];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) d[j * kMT + lane] = fp16_to_fp32((w[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+    }
     if constexpr (F == WFmt::Q4_1)  // the token's eight fp16 block sums, token-major
       *reinterpret_cast<uint4*>(&ast[slot][par][8 * lane]) = sraw;
   };
@@ -336,6 +344,12 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
     const uint8_t* AQ = stage;
     const uint8_t* wrow = stage + kAQ + (32 * wcol + col) * rl;
     const float* dxs = &adt[pair & 1][par][0];
+    const uint16_t* dq = reinterpret_cast<const uint16_t*>(dxs) + kMT * kg + col;  // kFactor
+    v16f qd[2];
+    auto add = [&](int t) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) y[t][r] = fmaf(qd[t][r], (float)I[t][r], y[t][r]);
+    };
     const uint16_t* sxs = &ast[pair & 1][par][0];
     // Q4_0: the row's 144 stage bytes as nine 16-byte LDS reads (the 36-dword
     // stride puts 16 lanes' 16-byte reads on all 64 banks); every record is
@@ -418,46 +432,53 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
         const uint32_t e = sh >= 1 ? ((w0 >> (8 * (sh - 1))) & 0xffu) : (ld32(wrow + b4 - 4) >> 24);
         wsc = scl[e];
       }
-      const uint32_t shn = 4 * kg;  // kg 0: elements 0..15 (low nibbles), 1: 16..31 (high)
-      uint32_t n[4] = {(q0 >> shn) & 0x0f0f0f0fu, (q1 >> shn) & 0x0f0f0f0fu,
-                       (q2 >> shn) & 0x0f0f0f0fu, (q3 >> shn) & 0x0f0f0f0fu};
+      // kg 0: elements 0..15 (low nibbles), 1: 16..31 (high).  Q4_0's nibbles
+      // go to the bytes' high halves with the top bit flipped, the int8
+      // 16 (q - 8) in a shift and one three-operand bit operation: y is summed
+      // as 16 y (a power of two, so exactly) and scaled at the end
+      const uint32_t shn = 4 * kg;
+      uint32_t n[4] = {q0, q1, q2, q3};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        n[i] = F == WFmt::Q4_0 ? ((n[i] << (4 - shn)) & 0xf0f0f0f0u) ^ 0x80808080u : (n[i] >> shn) & 0x0f0f0f0fu;
       v4i bv;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if constexpr (F == WFmt::Q4_0)
-          bv[i] = (int)(((n[i] | 0x80808080u) - 0x08080808u) ^ 0x80808080u);  // q - 8 per byte
+          bv[i] = (int)n[i];  // 16 (q - 8)
         else if constexpr (F == WFmt::Q4_1)
           bv[i] = (int)n[i];  // q in 0..15
         else
           bv[i] = (int)lookup16(n[i], c0, c1, c2, c3);
       }
       const int chunk = (2 * j + kg) ^ sw;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const v4i av = *reinterpret_cast<const v4i*>(AQ + (32 * t + col) * 256 + 16 * chunk);
-        I[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, zero, 0, 0, 0);
-      }
-      if constexpr (F == WFmt::Q4_0 || F == WFmt::Q4_1) {
+      if constexpr (kFactor) {
         // y += (dx dw) I with the factor dx dw of every output from one f16
         // MFMA per tile as an outer product: K slot 0 holds the token's dx
         // and the row's dw (both fp16, so each product is exact in fp32,
         // as the VALU product it replaces), every other slot 0
-        // (operands as raw bits: the kg half's slots are zero without a branch)
-        const uint32_t kmask = kg ? 0u : 0xffffu;
-        const v2u bq = {wbits & kmask, 0u};
+        // (operands as raw bits: the kg half reads the block's zeros).
+        // Tile 0's MFMAs run under the FMAs of the block before's tile 1, and
+        // tile 1's under tile 0's: with both tiles' MFMAs first, a wave stood
+        // still for their latency once a block.
+        const v2u bq = {wbits & (kg ? 0u : 0xffffu), 0u};
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          const _Float16 dxh = (_Float16)dxs[j * kMT + 32 * t + col];
-          const v2u aq = {(uint32_t)__builtin_bit_cast(uint16_t, dxh) & kmask, 0u};
-          const v16f qd = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, aq), __builtin_bit_cast(v4h, bq),
-                                                              fzero, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 16; ++r) y[t][r] = fmaf(qd[r], (float)I[t][r], y[t][r]);
+          const v4i av = *reinterpret_cast<const v4i*>(AQ + (32 * t + col) * 256 + 16 * chunk);
+          const v2u aq = {dq[2 * j * kMT + 32 * t], 0u};
+          I[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, zero, 0, 0, 0);
+          qd[t] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, aq), __builtin_bit_cast(v4h, bq),
+                                                      fzero, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (t == 1 || j > J0) add(1 - t);
         }
-        // keep the blocks' factor MFMAs in block order (hoisted, their
-        // results would hold registers across the whole stage)
-        __builtin_amdgcn_sched_barrier(0);
+        if (j == J0 + 3) add(1);
       } else {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const v4i av = *reinterpret_cast<const v4i*>(AQ + (32 * t + col) * 256 + 16 * chunk);
+          I[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, zero, 0, 0, 0);
+        }
         // y += (dx * ws) * I; register r of a tile holds token 8*(r/4) + 4*kg + r%4
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -508,6 +529,10 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
 
   issue(0, ring0);
   if (wcol == 0) {
+    if constexpr (kFactor)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        reinterpret_cast<uint16_t*>(&adt[i >> 3][par][0])[(2 * (i & 7) + 1) * kMT + lane] = 0;
     load_dx(0);
     store_dx(0);
   }
@@ -515,6 +540,12 @@ __device__ __forceinline__ void q80_gemm_body(const GemmArgs& a, uint8_t* lds) {
     step(pair, ring0, ring1);
     if (pair + 1 < npair) step(pair + 1, ring1, ring0);
   }
+
+  if constexpr (F == WFmt::Q4_0)  // summed as 16 y
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) y[t][r] *= 0.0625f;
 
   // both parities' partial sums -> two LDS planes (reusing the ring) -> Y
   __syncthreads();
