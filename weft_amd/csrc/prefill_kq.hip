@@ -412,9 +412,32 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     load_dx(0);
     dxq[0][lane] = bf16_split3(dxr);
   }
+  // Q6_K: the terms of four superblocks, then their sum into ysum with what
+  // that addition rounds off kept in ylow.  One chain over a row of 11008 values
+  // had twice the error of the GEMV's short ones (against 64 bits, relative:
+  // 1.3e-7, GEMV 0.70e-7; sums of eight without ylow 0.85e-7).
+  v16f ysum[2] = {}, ylow[2] = {};
+  auto fold = [&]() {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const v16f s = ysum[t] + y[t];
+      ylow[t] += (ysum[t] - s) + y[t];
+      ysum[t] = s;
+      y[t] = v16f{};
+    }
+  };
   for (int b = 0; b < nsb; b += 2) {
     step(b, ring0, 1, std::integral_constant<int, kOdd ? kRowShift : 0>{});
     if (b + 1 < nsb) step(b + 1, ring1, 0, std::integral_constant<int, kOdd ? kRowShift : k6 ? 2 : 0>{});
+    if (k6 && (b & 2)) fold();
+  }
+  if (k6) {
+    fold();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)  // an infinite sum leaves NaN in ylow
+        y[t][r] = ysum[t][r] + (fabsf(ysum[t][r]) < __builtin_huge_valf() ? ylow[t][r] : 0.f);
   }
 
   // both parities' partial sums -> two LDS planes (reusing the ring) -> Y

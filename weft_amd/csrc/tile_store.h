@@ -46,6 +46,11 @@ constexpr int kTilePlaneBytes = tile_plane_bytes<64, 128>();   // 34,816
 // bands are as even as they can be: a short last band would stream the
 // weights for few tokens.  Up to eight m-tiles the order is the plain one.
 __device__ inline void banded_tile(int t, int ntm, int ntn, int& tm, int& tn) {
+  if (ntm <= 8) {
+    tn = t / ntm;
+    tm = t - tn * ntm;
+    return;
+  }
   const int bands = (ntm + 7) >> 3, g = (ntm + bands - 1) / bands;
   const int band = t / (g * ntn), r = t - band * g * ntn;
   const int gm = min(g, ntm - band * g);
