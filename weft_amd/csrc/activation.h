@@ -258,15 +258,16 @@ __device__ inline void stage_q8k_load(const uint8_t* __restrict__ xq, int K, int
 
 // The end of a batch-1 GEMV whose rows are split into KS steps over KS waves:
 // rows [row_base, row_end) are their steps' partial sums (part[row - row_base]
-// [step]) added in step order.  Every thread of the workgroup calls it.
+// [step]) added in step order, in double: one rounding a row.  Every thread of
+// the workgroup calls it.
 template <int KS>
 __device__ __forceinline__ void gemv_add_steps(const float* part, float* Y, int row_base, int row_end) {
   __syncthreads();
   for (int r = threadIdx.x; r < row_end - row_base; r += blockDim.x) {
-    float y = part[r * KS];
+    double y = part[r * KS];
 #pragma unroll
     for (int s = 1; s < KS; ++s) y += part[r * KS + s];
-    Y[row_base + r] = y;
+    Y[row_base + r] = (float)y;
   }
 }
 
