@@ -705,7 +705,7 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
   for (int i = threadIdx.x; i < kOut; i += blockDim.x) {
     const int c = i & 15, row = 16 * (i >> 8) + 4 * ((i >> 4) & 3) + ((i >> 6) & 3);
     if (row >= mrows || n0 + c >= a.N) continue;
-    float v = 0.f;
+    double v = 0.;  // up to 16 sums: one rounding instead of one each
     for (int w = 0; w < nwaves; ++w) v += part[w * kOut + i];
     long long at;
     if constexpr (kGroup) {
@@ -714,7 +714,7 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
     } else {
       at = (long long)(m0 + row) * a.ldy;
     }
-    a.Y[at + n0 + c] = v;
+    a.Y[at + n0 + c] = (float)v;
   }
 }
 
