@@ -502,7 +502,7 @@ void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t
   gemm_iq2(W, Xq, grid, signs, Y, N, K, M, st);
 }
 
-// IQ2_XS: the same GEMM with per-half scales (M >= 16, K % 512 == 0), the GEMV otherwise
+// IQ2_XS: the same GEMM on scaled weights (K % 512 == 0), else the small-batch kernel or the GEMV
 void mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid, const int8_t* signs,
                     float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
   if (small_batch(7, W, X, Xq, grid, signs, Y, N, K, M, st)) return;

@@ -43,19 +43,20 @@ constexpr int kTilePlaneBytes = tile_plane_bytes<64, 128>();   // 34,816
 // blocks pass.  With all m-tiles of a column block in a row instead, 2048
 // tokens streamed the whole activation through every L2 for each column
 // block (11008 x 4096 weights: 0.95 GB of L2 misses a call for Q4_K).  The
-// bands are as even as they can be: a short last band would stream the
-// weights for few tokens.  Up to eight m-tiles the order is the plain one.
+// bands are even up to 24 m-tiles (a short last band would stream the weights
+// for few tokens; of more it is a small share).  Up to eight m-tiles the order
+// is the plain one.
 __device__ inline void banded_tile(int t, int ntm, int ntn, int& tm, int& tn) {
-  if (ntm <= 8) {
-    tn = t / ntm;
-    tm = t - tn * ntm;
-    return;
+  int m0 = 0, gm = ntm;
+  if (ntm > 8) {
+    const int g = ntm <= 16 ? (ntm + 1) / 2 : ntm <= 24 ? (ntm + 2) / 3 : 8;
+    const int band = t / (g * ntn);
+    t -= band * g * ntn;
+    m0 = band * g;
+    gm = min(g, ntm - m0);
   }
-  const int bands = (ntm + 7) >> 3, g = (ntm + bands - 1) / bands;
-  const int band = t / (g * ntn), r = t - band * g * ntn;
-  const int gm = min(g, ntm - band * g);
-  tn = r / gm;
-  tm = band * g + r - tn * gm;
+  tn = t / gm;
+  tm = m0 + t - tn * gm;
 }
 
 typedef float tile_v16f __attribute__((ext_vector_type(16)));
