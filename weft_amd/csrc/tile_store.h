@@ -45,7 +45,9 @@ constexpr int kTilePlaneBytes = tile_plane_bytes<64, 128>();   // 34,816
 // block (11008 x 4096 weights: 0.95 GB of L2 misses a call for Q4_K).  The
 // bands are even up to 24 m-tiles (a short last band would stream the weights
 // for few tokens; of more it is a small share).  Up to eight m-tiles the order
-// is the plain one.
+// is the plain one: one division, as every division here delays the first
+// loads (Q4_K 4096 x 4096, 512 rows, two calls: 0.5 us slower than without
+// bands where the band width took two more, 0.1 us now).
 __device__ inline void banded_tile(int t, int ntm, int ntn, int& tm, int& tn) {
   int m0 = 0, gm = ntm;
   if (ntm > 8) {
