@@ -647,8 +647,8 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
             for (int r = 0; r < 4; ++r) yt[r] = fmaf(f0 * dx[r], (float)I[r], yt[r]);
           } else if constexpr (F == SF::NVFP4) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              yt[r] = fmaf(dx[r] * f1, (float)I2[r], fmaf(dx[r] * f0, (float)I[r], yt[r]));
+            for (int r = 0; r < 4; ++r)  // a half's scale has four bits: its product with I is exact
+              yt[r] = fmaf(dx[r], fmaf(f1, (float)I2[r], f0 * (float)I[r]), yt[r]);
           } else {
             const float4 s4 = *reinterpret_cast<const float4*>(dxs + 128 * (MT + t) + 16 * s + 4 * q);
             const float xs[4] = {s4.x, s4.y, s4.z, s4.w};
