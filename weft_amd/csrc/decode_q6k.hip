@@ -46,10 +46,10 @@ struct Q6Args {
 // KS, wave w takes step w % KS (an even share of the superblocks, so its
 // activation slice still fits the registers) of the rows of group w / KS, and
 // the KS partial sums of a row are added in step order at the end.
-// One call, against the staged GEMV, whose rows all pass through LDS: 4096 x
-// 11008 (43 superblocks, 2-byte rows) 14.6 -> 13.1 us, 14336 x 5120 22.1 ->
-// 18.2, 2000 x 14336 13.2 -> 9.7.
-// kOdd: rows that are only 2-byte aligned, so a lane's shift is its row's.
+// One call, against the staged GEMV, whose rows all pass through LDS (weights
+// past the Infinity Cache): 4096 x 11008 (43 superblocks, 2-byte rows) 14.1 ->
+// 11.8 us, 14336 x 4352 20.1 -> 16.3, 1024 x 14336 10.8 -> 7.1.
+// kOdd: rows that are only 2-byte aligned, so a lane's shift depends on its row.
 template <int KS, bool kOdd>
 __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   constexpr int kGroups = kWaves / KS;
@@ -64,17 +64,19 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   const int sb = min(st * spb + (lane >> 2), nsb - 1), g = lane & 3, h = g >> 1;
   float* part = reinterpret_cast<float*>(lds + q8k_lds_row_bytes(K));  // [row - row_base][step]
   const uint32_t rec = (uint32_t)(kQ6_KBytes * sb);
-  // offset of the record from the dword holding its first byte (0 or 2); kOdd:
-  // row by row
-  const uint32_t sh_even = rec & 3u;
-  auto shift = [&](int row) -> uint32_t {
-    if constexpr (!kOdd) return sh_even;
-    return ((uint32_t)(uintptr_t)a.W + (uint32_t)row * (uint32_t)a.ldw + rec) & 2u;
+  // A row is read from the dword that holds its first byte, rbit (0 or 2) bytes
+  // before it: the row's address is then the wave's, and a lane's record lies
+  // `shift` (0 or 2) past the dword at its own offset `base`.  (With the shift
+  // taken from the lane's address instead, every row's loads need 64-bit
+  // addresses computed per lane, and the rows a wave
+  // has in flight fall behind: one call, weights past the Infinity Cache, 28672 x
+  // 4096 25.7 us where this takes 23.0, 4096 x 11008 12.4 and 11.8, 14336 x
+  // 16384 51.1 and 44.4.)
+  auto row_bit = [&](int row) -> uint32_t {
+    if constexpr (!kOdd) return 0u;
+    return ((uint32_t)(uintptr_t)a.W + (uint32_t)row * (uint32_t)a.ldw) & 2u;
   };
-  // the lane's regions, from the record's offset - sh on: ql [sh + 64h, +64), qh
-  // [sh + 128 + 32h, +32), scales [sh + 192 + 4g, +4), d [sh + 208, +2)
-  const uint32_t o_ql = rec + 64 * h, o_qh = rec + 128 + 32 * h, o_sc = rec + 192 + 4 * g;
-  const uint32_t o_d = rec + 208;
+  auto shift = [&](uint32_t rbit) -> uint32_t { return (rec + rbit) & 2u; };
   const size_t rb = a.ldw;
   const int row_base = blockIdx.x * a.rows_per_wg, row_first = row_base + grp;
   const int row_end = min(a.N, row_base + a.rows_per_wg);
@@ -85,30 +87,40 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   __builtin_amdgcn_sched_barrier(0);
 
   // 17 dwords of ql, 9 of qh, 2 of scales, 1 holding d.  A 17th / 9th /
-  // 2nd dword only carries data at sh = 2; at sh = 0 the last dword before it
+  // 2nd dword only carries data at a shift of 2; at 0 the last dword before it
   // is read again (the region may end at the row's end).
   struct RowBuf {
     uint32_t ql[17], qh[9], sc[2], d;
   };
   auto issue = [&](RowBuf& buf, int k) {
     const int row = min(row_first + k * kGroups, a.N - 1);  // clamped: always a valid row
-    const uint32_t sh = shift(row);
-    const uint8_t* rp = a.W + (size_t)row * rb - sh;
+    const uint32_t rbit = row_bit(row), sh = shift(rbit), base = rec + rbit - sh;
+    const uint8_t* rp = a.W + ((size_t)row * rb - rbit);
+    // the dword at o, at a shift of 2 the one after it (the two forms schedule
+    // differently: 14336 x 11008 32.6 us with the second one, 30.5 with the first;
+    // 4096 x 4096 2 % faster with the second)
+    auto last = [&](uint32_t o) {
+      if constexpr (kOdd)
+        return rp + (o + 2 * sh);
+      else
+        return rp + o + (sh ? 4 : 0);
+    };
+    const uint32_t o_ql = base + 64 * h, o_qh = base + 128 + 32 * h, o_sc = base + 192 + 4 * g;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(rp + o_ql + 16 * i);
       buf.ql[4 * i] = v.x, buf.ql[4 * i + 1] = v.y, buf.ql[4 * i + 2] = v.z, buf.ql[4 * i + 3] = v.w;
     }
-    buf.ql[16] = *reinterpret_cast<const uint32_t*>(rp + o_ql + (sh ? 64 : 60));
+    buf.ql[16] = *reinterpret_cast<const uint32_t*>(last(o_ql + 60));
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(rp + o_qh + 16 * i);
       buf.qh[4 * i] = v.x, buf.qh[4 * i + 1] = v.y, buf.qh[4 * i + 2] = v.z, buf.qh[4 * i + 3] = v.w;
     }
-    buf.qh[8] = *reinterpret_cast<const uint32_t*>(rp + o_qh + (sh ? 32 : 28));
+    buf.qh[8] = *reinterpret_cast<const uint32_t*>(last(o_qh + 28));
     buf.sc[0] = *reinterpret_cast<const uint32_t*>(rp + o_sc);
-    buf.sc[1] = *reinterpret_cast<const uint32_t*>(rp + o_sc + (sh ? 4 : 0));
-    buf.d = *reinterpret_cast<const uint32_t*>(rp + o_d);
+    buf.sc[1] = *reinterpret_cast<const uint32_t*>(last(o_sc));
+    buf.d = *reinterpret_cast<const uint32_t*>(rp + base + 208);
   };
   RowBuf bufA, bufB;
   issue(bufA, 0);
@@ -146,7 +158,7 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   const uint32_t hsh = 4 * (g & 1);        // qh bit pairs 2s: s = 2 (g & 1) and 2 (g & 1) + 1
 
   auto compute = [&](const RowBuf& buf, int k) {
-    const uint32_t sh = shift(row_first + k * kGroups);
+    const uint32_t sh = shift(row_bit(row_first + k * kGroups));
     uint32_t ql[16], qh[8];
 #pragma unroll
     for (int i = 0; i < 16; ++i) ql[i] = __builtin_amdgcn_alignbyte(buf.ql[i + 1], buf.ql[i], sh);  // sh 0 or 2
@@ -192,9 +204,12 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
 
   int k = 0;
   for (; k + 2 < nrows; k += 2) {
+    // (barriers: 28672 x 4096 24.6 -> 23.0 us; 4096 x 11008 11.6 -> 11.9, so not for kOdd)
     issue(bufB, k + 1);
+    if constexpr (!kOdd) __builtin_amdgcn_sched_barrier(0);
     compute(bufA, k);
     issue(bufA, k + 2);
+    if constexpr (!kOdd) __builtin_amdgcn_sched_barrier(0);
     compute(bufB, k + 1);
   }
   if (nrows - k == 2) {
