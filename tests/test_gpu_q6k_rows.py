@@ -55,3 +55,33 @@ def test_extreme_scales(hip, superblocks):
     G.mul_mat(s0, s1, G.tensor(G.F32, (n, m), yd.ptr), work.ptr, work.nbytes)
     hip.torch.cuda.synchronize()
     assert o.within_tolerance(yd.numpy(np.float32).reshape(m, n), e, a).all()
+
+
+def surrounded(hip, w, offset, fill):
+    """w on the GPU `offset` bytes past a 256-byte boundary, bytes `fill` around it."""
+    raw = np.full(w.nbytes + 512, fill, np.uint8)
+    raw[256 + offset:256 + offset + w.nbytes] = w.reshape(-1)
+    t = hip.torch.from_numpy(raw).to(hip.dev)
+    return t, t.data_ptr() + 256 + offset
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("n,k", [(1, 256), (3, 768), (33, 2816), (5, 11008), (4, 4096)])
+def test_batch1_reads_the_weights_alone(hip, n, k, offset):
+    """An odd number of records ends in the middle of a dword, and weights at
+    an address of 2 mod 4 begin in one.  The register kernel reads whole dwords
+    from a row's first one on, so it takes 4-byte aligned weights only; what lies
+    around the weights changes no bit of the result."""
+    from weft_amd import _lib
+    w, x = o.quantize("q6_k", o.seeded_normal(21, (n, k), 0.02)), o.seeded_normal(22, (1, k))
+    outs = []
+    for fill in (0x00, 0xFF):
+        keep, ptr = surrounded(hip, w, offset, fill)
+        xq, y = hip.empty(o.record_bytes("q8_k", k)), hip.empty(4 * n)
+        _lib.launch_log()
+        hip.call("production_mul_mat_q6_k_decode", ptr, hip.to_dev(x), xq, y, n, k, 1)
+        assert _lib.launch_log() == ["staged_gemv_kernel" if offset else "q6k_gemv_m1_kernel"]
+        outs.append(y.numpy(np.float32))
+    e, a = o.mul_mat_f64("q6_k", w, o.quantize("q8_k", x), n, k, 1)
+    assert o.within_tolerance(outs[0].reshape(1, n), e, a).all()
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))

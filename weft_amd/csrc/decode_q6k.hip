@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   // 16384 51.1 and 44.4.)
   auto row_bit = [&](int row) -> uint32_t {
     if constexpr (!kOdd) return 0u;
-    return ((uint32_t)(uintptr_t)a.W + (uint32_t)row * (uint32_t)a.ldw) & 2u;
+    return ((uint32_t)row * (uint32_t)a.ldw) & 2u;  // W itself is 4-byte aligned
   };
   auto shift = [&](uint32_t rbit) -> uint32_t { return (rec + rbit) & 2u; };
   const size_t rb = a.ldw;
@@ -86,9 +86,12 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   stager.prefetch(a.X, (size_t)K, K, 0, 1);
   __builtin_amdgcn_sched_barrier(0);
 
-  // 17 dwords of ql, 9 of qh, 2 of scales, 1 holding d.  A 17th / 9th /
-  // 2nd dword only carries data at a shift of 2; at 0 the last dword before it
-  // is read again (the region may end at the row's end).
+  // 17 dwords of ql, 9 of qh, 2 of scales, and d.  A 17th / 9th / 2nd dword
+  // only carries data at a shift of 2; at 0 the last dword before it is read
+  // again (the region may end at the row's end).  kOdd reads d by itself: as a
+  // dword at a shift of 0 it would reach two bytes past the record, and the last
+  // row's last record is the end of the weights.  (Rows of whole pairs of records
+  // end with one at a shift of 2, whose dword ends where the record does.)
   struct RowBuf {
     uint32_t ql[17], qh[9], sc[2], d;
   };
@@ -120,7 +123,10 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
     buf.qh[8] = *reinterpret_cast<const uint32_t*>(last(o_qh + 28));
     buf.sc[0] = *reinterpret_cast<const uint32_t*>(rp + o_sc);
     buf.sc[1] = *reinterpret_cast<const uint32_t*>(last(o_sc));
-    buf.d = *reinterpret_cast<const uint32_t*>(rp + base + 208);
+    if constexpr (kOdd)
+      buf.d = *reinterpret_cast<const uint16_t*>(rp + (rec + rbit + 208));
+    else
+      buf.d = *reinterpret_cast<const uint32_t*>(rp + base + 208);
   };
   RowBuf bufA, bufB;
   issue(bufA, 0);
@@ -165,7 +171,7 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) qh[i] = __builtin_amdgcn_alignbyte(buf.qh[i + 1], buf.qh[i], sh);
     const uint32_t sc4 = __builtin_amdgcn_alignbyte(buf.sc[1], buf.sc[0], sh);
-    const float dw = fp16_to_fp32((buf.d >> (8 * sh)) & 0xffffu);
+    const float dw = fp16_to_fp32(kOdd ? buf.d : (buf.d >> (8 * sh)) & 0xffffu);
     // part a: ql[0 .. 31] with qh bits hsh .. hsh + 1; part b: ql[32 .. 63]
     // with bits hsh + 2 .. hsh + 3 (element l of both parts reads qh[l])
     int P[4] = {0, 0, 0, 0};
@@ -237,14 +243,15 @@ void launch_steps(int ks, int grid, size_t lds, const Q6Args& a) {
 }  // namespace
 
 // Launches the kernel above when the call suits it: one activation row of
-// K <= 4 * 4096, 16-byte aligned X, W 2-byte aligned with rows a multiple of 2
-// bytes apart, Xq 4-byte aligned.
+// K <= 4 * 4096, 16-byte aligned X, W 4-byte aligned (of weights that begin in
+// the middle of a dword the first row would be read from before its first byte)
+// with rows a multiple of 2 bytes apart, Xq 4-byte aligned.
 bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st) {
   const size_t rb = K / 256 * kQ6_KBytes;
   const size_t ldw = N > 1 ? st.ldw : rb;
   if (N == 0 || K == 0 || K > 4 * 4096 || K % 256 != 0 || X == nullptr || Xq == nullptr || W == nullptr ||
-      Y == nullptr || !aligned(X, 16) || !aligned(W, 2) || ldw % 2 != 0 || !aligned(Y, 4) ||
+      Y == nullptr || !aligned(X, 16) || !aligned(W, 4) || ldw % 2 != 0 || !aligned(Y, 4) ||
       !aligned(Xq, 4) || N > (size_t)INT32_MAX || (N > 1 && ldw < rb) || ldw >= ((size_t)1 << 40))
     return false;
   const int cus = cu_count();
@@ -265,7 +272,7 @@ bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size
   const int grid = (int)((N + a.rows_per_wg - 1) / a.rows_per_wg);
   const size_t lds = q8k_lds_row_bytes((int)K) + (ks > 1 ? 4 * (size_t)ks * a.rows_per_wg : 0);
   if (lds > max_lds_per_block()) return false;
-  if (K % 512 != 0 || !aligned(W, 4) || ldw % 4 != 0)
+  if (K % 512 != 0 || ldw % 4 != 0)
     launch_steps<true>(ks, grid, lds, a);
   else
     launch_steps<false>(ks, grid, lds, a);
