@@ -85,3 +85,24 @@ def test_batch1_reads_the_weights_alone(hip, n, k, offset):
     e, a = o.mul_mat_f64("q6_k", w, o.quantize("q8_k", x), n, k, 1)
     assert o.within_tolerance(outs[0].reshape(1, n), e, a).all()
     np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("n,superblocks", [(33, 3), (129, 1), (5, 43)])
+def test_prefill_reads_the_weights_alone(hip, n, superblocks, offset):
+    """The GEMM's 2-byte rows, as the batch-1 kernel's: 4-byte aligned weights
+    only, and what lies around them changes no bit."""
+    from weft_amd import _lib
+    k, m = 256 * superblocks, 70
+    w, x = o.quantize("q6_k", o.seeded_normal(23, (n, k), 0.02)), o.seeded_normal(24, (m, k))
+    outs = []
+    for fill in (0x00, 0xFF):
+        keep, ptr = surrounded(hip, w, offset, fill)
+        xq, y = hip.empty(m * o.record_bytes("q8_k", k)), hip.empty(4 * m * n)
+        _lib.launch_log()
+        hip.call("production_mul_mat_q6_k", ptr, hip.to_dev(x), xq, y, n, k, m)
+        assert _lib.launch_log()[-1] == ("small_mfma_gemm" if offset else "q6k_mfma_gemm")
+        outs.append(y.numpy(np.float32).reshape(m, n))
+    e, a = o.mul_mat_f64("q6_k", w, o.quantize("q8_k", x), n, k, m)
+    assert o.within_tolerance(outs[0], e, a).all()
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))

@@ -117,6 +117,9 @@ __device__ __forceinline__ void lds_dma4(const uint8_t* g, uint32_t lds) {
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(lds_ptr)p;
 }
+__device__ __forceinline__ void lds_store16(uint32_t lds, uint32_t v) {
+  *reinterpret_cast<__attribute__((address_space(3))) uint16_t*>(lds) = (uint16_t)v;
+}
 __device__ __forceinline__ void pin(int& v) { asm volatile("" : "+v"(v)); }
 
 // 16 bytes that start sh (0 or 2) bytes past the 16-byte aligned LDS address
@@ -200,6 +203,25 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
   const bool w16 = ((reinterpret_cast<uintptr_t>(W) | wrb) & 15) == 0;  // Q5_K: 16-byte weight loads
   const uint32_t ring_lds[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(ring0)),
                                 (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(ring1))};
+  // (kOdd) the weights of the row's last superblock b where the tile holds the
+  // last row: of a record that begins with its dword, dword 52 ends two bytes
+  // past it, and past the last row's last one nothing may be read.  That row's
+  // d goes to its place (LDS bytes 220, 221) by itself.
+  auto issue_last = [&](int b, uint32_t base) {
+#pragma unroll 1
+    for (int k = wave; k < kNT * 15 / 64; k += 8) {
+      const int q = 64 * k + lane, row = q / 15, c = q - 15 * row, n = min(n0 + row, a.N - 1);
+      const uint8_t* g = W + (size_t)n * wrb + (size_t)b * TT::kRec;
+      const uint32_t gsh = (uint32_t)(uintptr_t)g & 2u;
+      const uint32_t at = base + kAQ + TT::kBS + 1024 * k;
+      if (n == a.N - 1 && gsh == 0 && c >= 13) {
+        const uint32_t d = *reinterpret_cast<const uint16_t*>(g + 208);
+        if (c == 13) lds_store16(at + 16 * lane + 12, d);
+      } else {
+        lds_dma16(g - gsh + min(16 * c, 196), at);
+      }
+    }
+  };
   auto issue = [&](int b, int slot) {
     const uint32_t base = ring_lds[slot];
 #pragma unroll
@@ -214,7 +236,9 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     if constexpr (k6) {
       // 15 chunks of 16 bytes a row (30 wave-wide loads, the row q / 15): 0 ..
       // 12 in place, 13 and 14 both the 16 bytes that end with dword 52, which
-      // so lands at bytes 220 .. 223 and nothing past it is read
+      // so lands at bytes 220 .. 223 and nothing past it is read (the weights'
+      // last record: issue_last)
+      if (kOdd && b + 1 == nsb && n0 + kNT >= a.N) return issue_last(b, base);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int k = wave + 8 * i;
@@ -456,10 +480,12 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
 
 // MFMA path: prefill shapes with 4-byte aligned weight rows, Q6_K also with
 // 2-byte aligned ones (kq_odd: a row of an odd number of 210-byte records
-// leaves the next one there).  The GEMV kernels take everything else.
+// leaves the next one there).  The weights themselves are 4-byte aligned: of
+// ones that are not, the first row would be read from before its first byte.
+// The small-batch kernel and the GEMVs take everything else.
 template <KQ F>
-bool kq_odd(const uint8_t* W, size_t ldw, size_t w_es, size_t K) {
-  return F == KQ::Q6_K && (K % 512 != 0 || !aligned(W, 4) || ldw % 4 != 0 || w_es % 4 != 0);
+bool kq_odd(size_t ldw, size_t w_es, size_t K) {
+  return F == KQ::Q6_K && (K % 512 != 0 || ldw % 4 != 0 || w_es % 4 != 0);
 }
 
 template <KQ F>
@@ -471,7 +497,7 @@ bool gemm_kq_ok(const uint8_t* W, const void* Xq, const float* Y, size_t N, size
   // below 16 activation rows only when the GEMV's LDS cannot hold a row
   return (M >= 16 || !staged_gemv_fits(F == KQ::Q6_K ? 3 : 4, K)) && N > 0 && K > 0 && K % 256 == 0 &&
          W != nullptr && Xq != nullptr && Y != nullptr &&
-         aligned(W, kAlign) && ldw % kAlign == 0 && aligned(Xq, 4) && aligned(Y, 4) && N <= (size_t)INT32_MAX &&
+         aligned(W, 4) && ldw % kAlign == 0 && aligned(Xq, 4) && aligned(Y, 4) && N <= (size_t)INT32_MAX &&
          K <= (size_t)INT32_MAX && M <= (size_t)INT32_MAX && strides_ok(st, K / 256 * kRec, 2, K, N, N, M) &&
          ((N + kNT - 1) / kNT) * ((M + kMT - 1) / kMT) <= (size_t)INT32_MAX;
 }
@@ -481,7 +507,7 @@ void gemm_kq(const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K, 
   const size_t ldw = N > 1 ? st.ldw : K / 256 * KTile<F>::kRec;
   GemmArgs ga{W, Xq, Y, (int)N, (int)K, (int)M, ldw, (long long)st.ldy, GroupTiles{}};
   const size_t tiles = ((N + kNT - 1) / kNT) * ((M + kMT - 1) / kMT);
-  if (kq_odd<F>(W, ldw, 0, K))
+  if (kq_odd<F>(ldw, 0, K))
     kq_mfma_gemm<false, F, F == KQ::Q6_K><<<dim3((unsigned)tiles), kThreads, 0, current_stream()>>>(ga);
   else
     kq_mfma_gemm<false, F><<<dim3((unsigned)tiles), kThreads, 0, current_stream()>>>(ga);
@@ -550,7 +576,7 @@ bool mul_mat_id_kq_grouped_ok(bool q6, const uint8_t* W, size_t xq_bytes, const 
   const size_t ldw = N > 1 ? st.ldw : rb;
   const size_t align = q6 ? 2 : 4;
   return N > 0 && n_pairs > 0 && K > 0 && K % 256 == 0 && W != nullptr && Y != nullptr &&
-         aligned(W, align) && ldw % align == 0 && aligned(Y, 4) && xq_bytes < ((size_t)1 << 32) && aligned(ws, 16) &&
+         aligned(W, 4) && ldw % align == 0 && aligned(Y, 4) && xq_bytes < ((size_t)1 << 32) && aligned(ws, 16) &&
          ws_bytes >= moe_group_bytes(n_pairs, pr.n_as) && pr.w_es % (long long)align == 0 && pr.n_as <= kMaxExperts &&
          N <= (size_t)INT32_MAX && K <= (size_t)INT32_MAX && strides_ok(st, rb, 2, K, N, N, 1) &&
          (size_t)moe_tile_bound(n_pairs, pr.n_as) * ((N + kNT - 1) / kNT) <= (size_t)INT32_MAX;
@@ -563,7 +589,7 @@ void mul_mat_id_kq_grouped(bool q6, const uint8_t* W, const uint8_t* Xq, float* 
   GemmArgs ga{W, Xq, Y, (int)N, (int)K, kMT, ldw, 0, group_tiles(g, pr)};
   const size_t wgs = (size_t)g.tmax * ((N + kNT - 1) / kNT);
   if (q6) {
-    if (kq_odd<KQ::Q6_K>(W, ldw, (size_t)pr.w_es, K))
+    if (kq_odd<KQ::Q6_K>(ldw, (size_t)pr.w_es, K))
       kq_mfma_gemm<true, KQ::Q6_K, true><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
     else
       kq_mfma_gemm<true, KQ::Q6_K><<<dim3((unsigned)wgs), kThreads, 0, current_stream()>>>(ga);
