@@ -41,3 +41,19 @@ def test_past_four_steps(hip, fmt):
 @pytest.mark.parametrize("k,pad", [(256, 0), (2816, 0), (1024, 2), (4096, 6), (11008, 4)])
 def test_q6k_two_byte_rows(hip, k, pad):
     assert launched(hip, "q6_k", k, 70, 1, pad_w=pad) == [KERNEL["q6_k"]]
+
+
+@pytest.mark.parametrize("n,k,kernel", [(14336, 12288, "staged_gemv_kernel"), (14335, 12288, KERNEL["q6_k"]),
+                                        (14336, 12032, KERNEL["q6_k"]), (14336, 12544, KERNEL["q6_k"])])
+def test_q6k_many_long_rows(hip, n, k, kernel):
+    """Many rows of three whole steps are the staged GEMV's (weights of zeros:
+    which kernel runs, and zeros out)."""
+    from weft_amd import _lib, ggml as G
+    w, x = hip.torch.zeros(n * k // 256 * 210, dtype=hip.torch.uint8, device=hip.dev), hip.empty(4 * k)
+    y, work = hip.empty(4 * n, fill=0xA5), hip.empty(k // 256 * 292)
+    _lib.launch_log()
+    G.mul_mat(G.tensor(G.Q6_K, (k, n), w.data_ptr()), G.tensor(G.F32, (k, 1), x.ptr),
+              G.tensor(G.F32, (n, 1), y.ptr), work.ptr, work.nbytes)
+    hip.torch.cuda.synchronize()
+    assert _lib.launch_log() == [kernel]
+    assert not y.numpy("float32").any()

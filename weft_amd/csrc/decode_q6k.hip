@@ -254,6 +254,11 @@ bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size
       Y == nullptr || !aligned(X, 16) || !aligned(W, 4) || ldw % 2 != 0 || !aligned(Y, 4) ||
       !aligned(Xq, 4) || N > (size_t)INT32_MAX || (N > 1 && ldw < rb) || ldw >= ((size_t)1 << 40))
     return false;
+  // The staged GEMV's 16-byte copies keep ahead of this kernel's per-lane reads
+  // where three or four whole steps a row and many rows leave nothing else to
+  // wait for: 14336 x 12288 32.7 us here, 32.0 there, 28672 x 16384 84.3 and
+  // 80.5 (equal at 11008 rows; rows of an odd number of records 5 % faster here).
+  if (K % 512 == 0 && K >= 3 * 4096 && N >= 14336) return false;
   const int cus = cu_count();
   const int ks = (int)((K + 4095) / 4096);
   const size_t groups = (size_t)(kWaves / ks);  // rows a workgroup works on at once
