@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from .test_gpu_ggml import FMTS, run, run_id
+from .test_gpu_ggml import FMTS, TYPE, make_weights, run, run_id
 
 pytestmark = pytest.mark.gpu
 
@@ -104,3 +104,54 @@ def test_many_rows_no_gemm_takes(hip, fmt, pad):
 def test_many_quantized_rows(hip, fmt):
     # a Q8_0 / Q8_1 src1, which those formats' GEMMs do not read
     assert launched(hip, fmt, 512, 75, 70, prequant=True) == ["small_mfma_gemm"]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("m", [5, 20])
+def test_values_that_are_not_finite(hip, fmt, m):
+    """Activations and weight scales at and past the ends of fp16: outputs are
+    NaN, inf (and of which sign) and finite where GGML's are, the finite ones
+    within the usual bound.  (Q4_K, Q5_K and Q6_K, whose superblocks GGML sums in
+    eight parts, so that an infinite scale gives infinities of both signs: finite
+    where GGML's are.)"""
+    from weft_amd import _lib, ggml as G
+    n, k = 48, 768
+    rng = np.random.default_rng(31)
+    w = make_weights(fmt, n, k, 5).copy()
+    x = o.seeded_normal(6, (m, k))
+    act = o.ACT_OF[fmt]
+    if act == "q8_k":
+        x[1, 256:512] *= 1e20
+    else:
+        x[1, 64:96] *= 1e8      # the block's fp16 scale is inf
+        x[2, 64:96] = 0.0
+        x[2, 65] = 1e8          # ... with one value that is not 0
+        x[3] = 0.0              # an all-zero token
+    if fmt != "mxfp4" and fmt != "nvfp4":
+        elems, nbytes = (256, o.record_bytes(fmt, 256)) if act == "q8_k" else (32, o.record_bytes(fmt, 32))
+        rec = w.reshape(n, k // elems, nbytes)
+        at = 208 if fmt == "q6_k" else 0
+        for row, bits in ((3, 0x7C00), (4, 0xFC00), (5, 0x7BFF), (6, 0x0001), (7, 0x0000)):
+            rec[row, 1, at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    else:
+        for row in range(8, 12):  # rows with zero scales and zero codes
+            w[row] = w[row] * (rng.random(w.shape[1]) < 0.7)
+    xq = o.quantize(act, x)
+    g = o.mul_mat_q(fmt, w, xq, n, k, m)
+    e, a = o.mul_mat_f64(fmt, w, xq, n, k, m)
+    wd, xd, yd = hip.to_dev(w), hip.to_dev(x), hip.empty(4 * n * m)
+    s0, s1 = G.tensor(TYPE[fmt], (k, n), wd.ptr), G.tensor(G.F32, (k, m), xd.ptr)
+    work = hip.empty(G.mul_mat_work_size(s0, s1))
+    _lib.launch_log()
+    G.mul_mat(s0, s1, G.tensor(G.F32, (n, m), yd.ptr), work.ptr, work.nbytes)
+    hip.torch.cuda.synchronize()
+    assert "small_mfma_gemm" in _lib.launch_log()
+    y = yd.numpy(np.float32).reshape(m, n)
+    assert (~np.isfinite(g)).any() and np.isfinite(g).any()
+    np.testing.assert_array_equal(np.isfinite(y), np.isfinite(g))
+    if fmt in ("q4_k", "q5_k", "q6_k"):
+        y, g = np.where(np.isfinite(y), y, np.nan), np.where(np.isfinite(g), g, np.nan)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(g))
+    np.testing.assert_array_equal(np.where(np.isinf(y), np.sign(y), 0), np.where(np.isinf(g), np.sign(g), 0))
+    fin = np.isfinite(g)
+    assert o.within_tolerance(y[fin], g[fin].astype(np.float64), a[fin]).all()

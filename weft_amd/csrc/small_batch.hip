@@ -581,6 +581,8 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
       fetch_w(u + nwaves);
     }
     wave_lds_fence();
+    // NVFP4: whether a token's block scale of the unit is not finite
+    bool odd_dx = false;
     if constexpr (!T::kQ8K) {
       // the tokens' block scales as floats: lane (token col, blocks q, q + 4)
 #pragma unroll
@@ -588,12 +590,15 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int at = (16 * t + col) * T::kXPitch + (q + 4 * i) * T::kXRec;
-          dxs[128 * t + 16 * (q + 4 * i) + col] = fp16_to_fp32(half_at(xwin, at));
+          const uint32_t d = half_at(xwin, at);
+          dxs[128 * t + 16 * (q + 4 * i) + col] = fp16_to_fp32(d);
+          if constexpr (F == SF::NVFP4) odd_dx |= 16 * t + col < mrows && (d & 0x7c00u) == 0x7c00u;
           if constexpr (T::kAct == Act::Q8_1)
             dxs[128 * (MT + t) + 16 * (q + 4 * i) + col] = fp16_to_fp32(half_at(xwin, at + 2));
         }
     }
     if constexpr (!T::kQ8K) wave_lds_fence();
+    if constexpr (F == SF::NVFP4) odd_dx = __builtin_amdgcn_ballot_w64(odd_dx) != 0;
     const int xo = col * T::kXPitch + 8 * q, o = col * T::kPitch;
     Row<F> row;
     row.begin(win, o, ext + 16 * col, sh);
@@ -606,7 +611,8 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
         S[t][r] = 0;
         yu[t][r] = 0.f;
       }
-    for_blocks([&](auto blk) {
+    // one block's terms; apart (NVFP4): each half's by itself, in GGML's order
+    auto block_terms = [&](auto blk, auto apart) {
       constexpr int s = decltype(blk)::value;
       long x[MT];
 #pragma unroll
@@ -646,9 +652,17 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
 #pragma unroll
             for (int r = 0; r < 4; ++r) yt[r] = fmaf(f0 * dx[r], (float)I[r], yt[r]);
           } else if constexpr (F == SF::NVFP4) {
+            if constexpr (decltype(apart)::value) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)  // a half's scale has four bits: its product with I is exact
-              yt[r] = fmaf(dx[r], fmaf(f1, (float)I2[r], f0 * (float)I[r]), yt[r]);
+              for (int r = 0; r < 4; ++r)
+                yt[r] = ggml_scaled_term(ggml_scaled_term(yt[r], dx[r], f0, (float)I[r]), dx[r], f1, (float)I2[r]);
+            } else {
+              // a UE4M3 scale has four bits, so its product with I is exact (of a
+              // caller's table: rounded once)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                yt[r] = fmaf(dx[r], fmaf(f1, (float)I2[r], f0 * (float)I[r]), yt[r]);
+            }
           } else {
             const float4 s4 = *reinterpret_cast<const float4*>(dxs + 128 * (MT + t) + 16 * s + 4 * q);
             const float xs[4] = {s4.x, s4.y, s4.z, s4.w};
@@ -659,7 +673,17 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
           for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(yt[r]));
         }
       }
-    });
+    };
+    // Where a token's scale is not finite (NVFP4): an infinite dx is NaN with a
+    // half that is zero and with two halves of unlike signs (ggml-cpu/quants.c:
+    // 279-313), which the sum of the halves would hide.  A loop of its own, as a
+    // choice at every block made every call 3 to 9 % longer.
+    bool apart = false;
+    if constexpr (F == SF::NVFP4) {
+      apart = odd_dx;
+      if (apart) for_blocks([&](auto blk) { block_terms(blk, std::true_type{}); });
+    }
+    if (!apart) for_blocks([&](auto blk) { block_terms(blk, std::false_type{}); });
     if constexpr (T::kQ8K) {
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
