@@ -155,3 +155,27 @@ def test_values_that_are_not_finite(hip, fmt, m):
     np.testing.assert_array_equal(np.where(np.isinf(y), np.sign(y), 0), np.where(np.isinf(g), np.sign(g), 0))
     fin = np.isfinite(g)
     assert o.within_tolerance(y[fin], g[fin].astype(np.float64), a[fin]).all()
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k"])
+@pytest.mark.parametrize("m", [3, 15])
+def test_any_bsums(hip, fmt, m):
+    """A Q8_K src1 whose bsums are a caller's own, up to the ends of int16 and
+    not the sums of its values (which are at most 2048): they are taken as they
+    are, as GGML's vec_dot does."""
+    from weft_amd import ggml as G
+    n, k = 40, 1024
+    rng = np.random.default_rng(33)
+    w = make_weights(fmt, n, k, 34)
+    xq = o.quantize("q8_k", o.seeded_normal(35, (m, k))).reshape(m, k // 256, 292)
+    bs = rng.integers(-32768, 32768, size=(m, k // 256, 16)).astype(np.int16)
+    bs[0, 0], bs[0, 1], bs[1, 0] = -32768, 32767, 2049
+    xq[:, :, 260:] = bs.view(np.uint8).reshape(m, k // 256, 32)
+    xq = np.ascontiguousarray(xq.reshape(m, -1))
+    want = o.mul_mat_q(fmt, w, xq, n, k, m)
+    wd, xd, yd = hip.to_dev(w), hip.to_dev(xq), hip.empty(4 * n * m)
+    G.mul_mat(G.tensor(TYPE[fmt], (k, n), wd.ptr), G.tensor(G.Q8_K, (k, m), xd.ptr), G.tensor(G.F32, (n, m), yd.ptr))
+    hip.torch.cuda.synchronize()
+    y = yd.numpy(np.float32).reshape(m, n)
+    # fp32 sums of the same integers: eight roundings a superblock of GGML's 1 / 2 ulp, and this kernel's
+    assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max()

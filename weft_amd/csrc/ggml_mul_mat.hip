@@ -458,7 +458,7 @@ hipError_t mul_mat_id(const weft_ggml_tensor* s0, const weft_ggml_tensor* s1,
                   : vd->size == kQ8_1Bytes ? quantize_q8_1_rows
                                            : quantize_q8_0_rows);
     small_pairs(gemv_format(s0->type), W, xq, tables0(tab, s0->type), tables1(tab, s0->type), Y, (size_t)N, (size_t)K,
-                st, pr, n_pairs);
+                st, pr, n_pairs, !quantize);
     return pending_error();
   }
   // several pairs per expert on average, or rows the pair GEMV cannot hold

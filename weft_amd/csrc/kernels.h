@@ -228,12 +228,13 @@ bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const i
                            float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm = true);
 // MUL_MAT_ID's (token, slot) pairs on the same kernel, 2 .. 64 of them, which
 // groups them by expert itself: Xq holds the x_rows quantized src1 rows
-// (token * ne11 + row).  _ok: whether the shape suits it.
+// (token * ne11 + row), caller_xq: as the caller made them (their bsums may
+// then be any int16).  _ok: whether the shape suits it.
 bool small_pairs_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
                     const float* Y, size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs,
                     size_t x_rows);
 void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1, float* Y,
-                 size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs);
+                 size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs, bool caller_xq);
 
 // Activation quantizers over K contiguous values, and over M rows of K
 // values ldx floats apart (records written contiguously).

@@ -45,6 +45,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // as decode_quantized's format codes, and Q4_K
 enum class SF { Q4_0, MXFP4, IQ2_XXS, Q6_K, Q5_K, NVFP4, Q4_1, IQ2_XS, Q4_K };
@@ -106,6 +107,7 @@ struct Args {
   long long ldy;    // floats between output rows
   PairArgs pair;    // MUL_MAT_ID mode: at most 64 pairs
   int n_pairs;
+  bool wide;        // Xq is the caller's own
 };
 
 // chunk loads per lane of 16 rows
@@ -377,8 +379,10 @@ __device__ __forceinline__ void for_blocks(Fn f) {
   f(std::integral_constant<int, 7>{});
 }
 
-// MT token tiles of 16
-template <SF F, int MT, bool kGroup>
+// MT token tiles of 16.  kWide (Q4_K, Q5_K): a caller's Q8_K records, whose
+// bsums may be any int16; a quantizer's are at most 2048, exact in f16 (the
+// wide form makes calls 1 to 7 % longer)
+template <SF F, int MT, bool kGroup, bool kWide>
 __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args a) {
   using T = Traits<F>;
   static_assert(T::kTableBytes + 64 + max_waves<MT>() * wave_lds<F, MT>() <= 158 * 1024, "fits the LDS");
@@ -694,13 +698,25 @@ __global__ void __launch_bounds__((64 * max_waves<MT>())) small_gemm_kernel(Args
           // Mn = sum_j m_{j/2} bsum_j: exact in f16 operands and fp32 sums
           uint32_t bs[2];  // bsums 4 q .. + 3 of token col
           run<256>(xwin, xo + 16 * t * T::kXPitch, bs);
-          const v4h am = {(_Float16)(short)(bs[0] & 0xffffu), (_Float16)(short)(bs[0] >> 16),
-                          (_Float16)(short)(bs[1] & 0xffffu), (_Float16)(short)(bs[1] >> 16)};
           const uint32_t mw = (q < 2 ? row.mn03 : row.mn47) >> (16 * (q & 1));
           const _Float16 ma = (_Float16)(float)(mw & 63u), mb = (_Float16)(float)((mw >> 8) & 63u);
-          const v4h bm = {ma, ma, mb, mb};
+          const short b[4] = {(short)(bs[0] & 0xffffu), (short)(bs[0] >> 16), (short)(bs[1] & 0xffffu),
+                              (short)(bs[1] >> 16)};
           const v4f fz = {};
-          const v4f mn = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, fz, 0, 0, 0);
+          v4f mn;
+          if constexpr (kWide) {
+            // as 16 hi + lo in two of 32 places: lo's mins are m, hi's 16 m (at most 1008)
+            const v8h am = {(_Float16)(short)(b[0] & 15), (_Float16)(short)(b[1] & 15), (_Float16)(short)(b[2] & 15),
+                            (_Float16)(short)(b[3] & 15), (_Float16)(short)(b[0] >> 4), (_Float16)(short)(b[1] >> 4),
+                            (_Float16)(short)(b[2] >> 4), (_Float16)(short)(b[3] >> 4)};
+            const _Float16 k16 = (_Float16)16.f;
+            const v8h bm = {ma, ma, mb, mb, k16 * ma, k16 * ma, k16 * mb, k16 * mb};
+            mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm, fz, 0, 0, 0);
+          } else {
+            const v4h am = {(_Float16)b[0], (_Float16)b[1], (_Float16)b[2], (_Float16)b[3]};
+            const v4h bm = {ma, ma, mb, mb};
+            mn = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, fz, 0, 0, 0);
+          }
 #pragma unroll
           for (int r = 0; r < 4; ++r) yt[r] = fmaf(dx[r], row.dw * (float)S[t][r] - row.dmin * mn[r], yt[r]);
         } else {
@@ -755,8 +771,12 @@ void launch_tile(const Args& a, int gx, int gy) {
   nwaves = std::min(nwaves, a.K / 256);  // every wave has a unit
   const size_t bytes = std::max((size_t)Traits<F>::kTableBytes + (size_t)nwaves * wave_lds<F, MT>(),
                                 (size_t)nwaves * MT * 1024);
-  small_gemm_kernel<F, MT, kGroup>
-      <<<dim3((unsigned)gx, (unsigned)gy), nwaves * kWave, bytes, current_stream()>>>(a);
+  const dim3 grid((unsigned)gx, (unsigned)gy);
+  constexpr bool kBsums = F == SF::Q4_K || F == SF::Q5_K;
+  if (kBsums && a.wide)
+    small_gemm_kernel<F, MT, kGroup, kBsums><<<grid, nwaves * kWave, bytes, current_stream()>>>(a);
+  else
+    small_gemm_kernel<F, MT, kGroup, false><<<grid, nwaves * kWave, bytes, current_stream()>>>(a);
   check_launch(kGroup ? "small_mfma_gemm_grouped" : "small_mfma_gemm");
 }
 
@@ -867,15 +887,19 @@ static bool small_wins(int fmt, size_t N, size_t M, bool gemm) {
   return w <= (fmt == 8 && M > 32 ? kLimit[fmt] * 3u / 2u : kLimit[fmt]);
 }
 
-bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
-                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm) {
+static bool small_run(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
+                      float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm, bool wide) {
   if (!small_wins(fmt, N, M, gemm) || st.ldy < N || st.ldy >= ((size_t)1 << 38) ||
       !small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, M, st)) return false;
   const FmtInfo f = fmt_info(fmt);
   const Args a{W, Xq, tab0, tab1, Y, (int)N, (int)K, (int)M, 1, (uint32_t)(N > 1 ? st.ldw : K / f.elems * f.rec),
-               (long long)st.ldy, PairArgs{}, 0};
+               (long long)st.ldy, PairArgs{}, 0, wide};
   launch_fmt(fmt, a);
   return true;
+}
+bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
+                           float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm) {
+  return small_run(fmt, W, Xq, tab0, tab1, Y, N, K, M, st, gemm, true);
 }
 
 bool small_pairs_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
@@ -885,10 +909,10 @@ bool small_pairs_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* 
          small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, x_rows, st);
 }
 void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1, float* Y,
-                 size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs) {
+                 size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs, bool caller_xq) {
   const FmtInfo f = fmt_info(fmt);
   const Args a{W, Xq, tab0, tab1, Y, (int)N, (int)K, 16, 1, (uint32_t)(N > 1 ? st.ldw : K / f.elems * f.rec),
-               0, pr, n_pairs};
+               0, pr, n_pairs, caller_xq};
   launch_fmt(fmt, a);
 }
 
@@ -904,7 +928,7 @@ bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const i
     case 6: quantize_q8_1_rows(X, st.ldx, Xq, M, K); break;
     default: quantize_q8_k_rows(X, st.ldx, Xq, M, K); break;
   }
-  return small_batch_quantized(fmt, W, Xq, tab0, tab1, Y, N, K, M, st, gemm);
+  return small_run(fmt, W, Xq, tab0, tab1, Y, N, K, M, st, gemm, false);
 }
 
 }  // namespace weft
