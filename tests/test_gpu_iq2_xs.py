@@ -141,3 +141,18 @@ def test_decode_iq2_xs_batch1_extreme_records(hip):
     x[0, 256:512] = 0.0
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_iq2_xs", "iq2_xs", n, k, 1, w=w, x=x)
     check_mul_mat("iq2_xs", w, x, xq, y, n, k, 1)
+
+
+@pytest.mark.parametrize("m", [1, 4, 15])
+def test_staged_name_is_the_same_call(hip, m):
+    """production_mul_mat_iq2_xs and its _staged name run the same kernels at
+    every M: the same launches, the same bits."""
+    n, k = 200, 1024
+    outs, names = [], []
+    for symbol in ("production_mul_mat_iq2_xs", "production_mul_mat_iq2_xs_staged"):
+        hip._lib.launch_log()
+        outs.append(run_mul_mat(hip, symbol, "iq2_xs", n, k, m, w=weights(n, k))[3])
+        names.append(hip._lib.launch_log())
+    assert names[0] == names[1]
+    assert ("small_mfma_gemm" in names[0]) == (m > 1), names
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))

@@ -66,17 +66,13 @@ void production_mul_mat_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, floa
 void production_mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid,
                                const int8_t* signs, float* Y, size_t N, size_t K, size_t M) {
   if (X == nullptr || Xq == nullptr) return weft::set_error(hipErrorInvalidValue);
-  const weft::RowStrides st = weft::packed(K / 256 * weft::kIq2xsBytes, K, N);
-  // the reference has no _decode symbol for this format: a few rows take the GEMV here
-  if (M < 16) return weft::decode_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, st);
-  weft::mul_mat_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, st);
+  weft::mul_mat_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, weft::packed(K / 256 * weft::kIq2xsBytes, K, N));
 }
 
 void production_mul_mat_iq2_xs_staged(const uint8_t* W, const float* X, uint8_t* Xq,
                                       const int8_t* grid, const int8_t* signs, float* Y, size_t N,
                                       size_t K, size_t M) {
-  if (X == nullptr || Xq == nullptr) return weft::set_error(hipErrorInvalidValue);
-  weft::mul_mat_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M, weft::packed(K / 256 * weft::kIq2xsBytes, K, N));
+  production_mul_mat_iq2_xs(W, X, Xq, grid, signs, Y, N, K, M);
 }
 
 void production_mul_mat_mxfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
