@@ -179,3 +179,13 @@ def test_any_bsums(hip, fmt, m):
     y = yd.numpy(np.float32).reshape(m, n)
     # fp32 sums of the same integers: eight roundings a superblock of GGML's 1 / 2 ulp, and this kernel's
     assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("fmt,n,k,m", [
+    ("q4_0", 4090, 2304, 20), ("q4_0", 4112, 2304, 20),    # eight waves; 257 workgroups: four
+    ("q4_0", 12288, 1024, 17), ("q4_0", 12304, 1024, 17),  # four waves; 769 workgroups: two
+    ("q4_1", 8208, 1280, 33), ("q5_k", 12304, 768, 20),    # two waves, uneven shares of the units
+])
+def test_waves_of_a_workgroup(hip, fmt, n, k, m):
+    """Each choice of the waves that share K, on both sides of where it changes."""
+    assert "small_mfma_gemm" in launched(hip, fmt, k, n, m)

@@ -764,13 +764,25 @@ void launch_tile(const Args& a, int gx, int gy) {
   // two workgroups, else twice as many per halving, so that about eight waves
   // a CU load at once.  Measured, Q4_K, 8 tokens: 11008 x 4096 (688
   // workgroups) 13.4 / 13.7 / 16.6 us a call at 4 / 8 / 16 waves, 4096 x 4096
-  // (256) 10.2 / 8.1 / 8.1.
+  // (256) 10.2 / 8.1 / 8.1.  (MUL_MAT_ID's count is of all pairs, though of
+  // those of one expert only one in sixteen works: the others are launched too.)
+  // All of them at the same time, though: with two token tiles a CU's LDS holds
+  // one workgroup of eight waves, three of four and six of two, and a second
+  // round costs as much as the first.  So eight waves only where every
+  // workgroup has a CU (Q4_K, 32 tokens, 5120 x 4096: 15.1 us at eight, 13.9 at
+  // four), and two where four leave a rest that two do not, up to 3072 values
+  // (IQ2_XXS, 32 tokens, 16384 x 1536: 17.4 us at four, 14.2 at two; at 11008
+  // values two are up to 15 % slower).
   const int wgs = gx * gy;
+  auto lds_bytes = [](int waves) { return (size_t)Traits<F>::kTableBytes + (size_t)waves * wave_lds<F, MT>(); };
+  auto one_round = [&](int waves) {
+    return (size_t)wgs <= (size_t)cu_count() * (160 * 1024 / (lds_bytes(waves) + 64));
+  };
   int nwaves = 4;
-  while (nwaves < max_waves<MT>() && wgs * nwaves < 8 * cu_count()) nwaves *= 2;
+  while (nwaves < max_waves<MT>() && wgs * nwaves < 8 * cu_count() && one_round(2 * nwaves)) nwaves *= 2;
+  if (MT == 2 && a.K <= 3072 && !one_round(4) && one_round(2)) nwaves = 2;
   nwaves = std::min(nwaves, a.K / 256);  // every wave has a unit
-  const size_t bytes = std::max((size_t)Traits<F>::kTableBytes + (size_t)nwaves * wave_lds<F, MT>(),
-                                (size_t)nwaves * MT * 1024);
+  const size_t bytes = std::max(lds_bytes(nwaves), (size_t)nwaves * MT * 1024);
   const dim3 grid((unsigned)gx, (unsigned)gy);
   constexpr bool kBsums = F == SF::Q4_K || F == SF::Q5_K;
   if (kBsums && a.wide)
