@@ -147,7 +147,7 @@ def test_decode_iq2_xs_batch1_extreme_records(hip):
 def test_staged_name_is_the_same_call(hip, m):
     """production_mul_mat_iq2_xs and its _staged name run the same kernels at
     every M: the same launches, the same bits."""
-    n, k = 200, 1024
+    n, k = 200, 4096
     outs, names = [], []
     for symbol in ("production_mul_mat_iq2_xs", "production_mul_mat_iq2_xs_staged"):
         hip._lib.launch_log()

@@ -23,8 +23,9 @@ def launched(hip, *args, **kwargs):
 @pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("m", [4, 15, 16, 17, 32, 33, 64])
 def test_token_tiles(hip, fmt, m):
-    # 2 and 5 units over 4 .. 8 waves, a partial weight tile
-    names = launched(hip, fmt, 512 if m % 2 else 1280, 75, m)
+    # 2 and 5 units over 4 .. 8 waves, a partial weight tile (4 rows: the shortest
+    # values of one GEMV pass that the kernel takes)
+    names = launched(hip, fmt, 4096 if m == 4 else 512 if m % 2 else 1280, 75, m)
     assert "small_mfma_gemm" in names, names
 
 
@@ -36,8 +37,44 @@ def test_weight_tiles_and_long_rows(hip, fmt, n, units):
 
 @pytest.mark.parametrize("fmt,first", [("q4_k", 2), ("q5_k", 2), ("q4_0", 3), ("mxfp4", 4), ("nvfp4", 4)])
 def test_fewest_rows(hip, fmt, first):
-    assert "small_mfma_gemm" in launched(hip, fmt, 512, 64, first)
-    assert not any("gemm" in name for name in launched(hip, fmt, 512, 64, first - 1))
+    assert "small_mfma_gemm" in launched(hip, fmt, 4096, 4096, first)
+    assert not any("gemm" in name for name in launched(hip, fmt, 4096, 4096, first - 1))
+
+
+@pytest.mark.parametrize("fmt,m,k,n,small", [
+    ("q4_0", 3, 1024, 64, False), ("q5_k", 2, 1024, 64, False), ("q6_k", 4, 2048, 64, False),
+    ("iq2_xs", 4, 256, 40, False), ("q4_1", 4, 3840, 64, False), ("q4_1", 4, 4096, 64, True),
+    ("q4_0", 3, 1024, 8191, False), ("q4_0", 3, 1024, 8192, True),
+    ("q5_k", 4, 1024, 4096, True), ("q5_k", 4, 1024, 4095, False), ("q4_1", 4, 1024, 4096, False),
+    ("q4_k", 2, 256, 16, True), ("q4_0", 5, 256, 16, True),
+])
+def test_one_gemv_pass(hip, fmt, m, k, n, small):
+    """A short batch of one GEMV pass stays one launch; more rows, and Q4_K's
+    longer pass, take the kernel, as does a quantized src1."""
+    assert ("small_mfma_gemm" in launched(hip, fmt, k, n, m)) == small
+    if m >= 4:
+        assert launched(hip, fmt, k, n, m, prequant=True) == ["small_mfma_gemm"]
+
+
+@pytest.mark.parametrize("fmt,m,k,n,small", [
+    ("q4_k", 32, 2048, 4096, True), ("q4_k", 32, 2048, 4097, False), ("q4_k", 17, 2304, 4097, True),
+    ("q4_k", 33, 256, 6144, True), ("q4_k", 33, 256, 6145, False), ("q4_k", 16, 256, 13108, True),
+    ("q4_k", 16, 256, 13109, False), ("mxfp4", 20, 256, 14000, True), ("mxfp4", 20, 256, 14001, False),
+    ("mxfp4", 20, 3328, 12288, True), ("mxfp4", 20, 3328, 12289, False),
+])
+def test_most_rows(hip, fmt, m, k, n, small):
+    """Both sides of the limits to the prefill GEMM (weights of zeros: which
+    kernel runs, and zeros out)."""
+    from weft_amd import _lib, ggml as G
+    w = hip.torch.zeros(n * o.record_bytes(fmt, k), dtype=hip.torch.uint8, device=hip.dev)
+    x, y = hip.empty(4 * m * k), hip.empty(4 * m * n, fill=0xA5)
+    s0, s1 = G.tensor(TYPE[fmt], (k, n), w.data_ptr()), G.tensor(G.F32, (k, m), x.ptr)
+    work = hip.empty(G.mul_mat_work_size(s0, s1))
+    _lib.launch_log()
+    G.mul_mat(s0, s1, G.tensor(G.F32, (n, m), y.ptr), work.ptr, work.nbytes)
+    hip.torch.cuda.synchronize()
+    assert ("small_mfma_gemm" in _lib.launch_log()) == small
+    assert not y.numpy(np.float32).any()
 
 
 @pytest.mark.parametrize("fmt", FMTS)

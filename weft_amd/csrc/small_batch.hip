@@ -876,32 +876,53 @@ static bool small_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t*
          tables_ok(fmt, tab0, tab1) && strides_ok(st, K / f.elems * f.rec, f.w_align, K, N, N, 1);
 }
 
-// Whether the small-batch kernel is the faster one.  Below 16 rows the other
-// is a GEMV of four rows a pass, with the quantization in the same launch:
-// Q4_K / Q5_K win from 2 rows (11008 x 4096: 11.9 against 13.8 us, 12.6
-// against 14.1), the rest from 3 (Q4_0 13.7 against 14.9; at 2, 13.6 against
-// 12.7), MXFP4 and the formats with two scales a block from 4 (NVFP4 18.3
-// against 17.0 at 3).  From 16 rows it is the prefill GEMM, which takes
-// one K loop of a 64 x 128 tile whatever N is until the tiles fill the chip,
-// while this kernel's time grows with the weight rows times the token tiles;
-// both grow with K.  The limits are where the two lines measured at 4096 and
-// 11008 x 4096, 16 .. 64 rows, cross (MXFP4, 64 rows: 20.7 against 33.0 us
-// at 4096 rows, 41.0 against 35.3 at 11008).
-static bool small_wins(int fmt, size_t N, size_t M, bool gemm) {
+// Whether the small-batch kernel is the faster one (figures: one call, replayed
+// from a graph).
+//
+// Below 16 rows the other is a GEMV of four rows a pass, with the quantization
+// in the same launch.  A batch of one pass is that one launch against two, about
+// 4 against 7 us of host time where both are short, until the pass is longer:
+// from 28M products of weights and rows on (Q4_0, 3 rows: 2048 x 2048 5.6 against
+// 6.2 us, 4096 x 2048 6.2 against 6.1, 4096 x 4096 8.9 against 8.3), from 16M
+// where it is long itself (Q5_K, Q6_K, NVFP4: Q5_K, 4 rows, 4096 x 1024 7.1
+// against 5.6), of 16384 activation values, which every workgroup quantizes (Q4_0,
+// 4 rows, 64 x 4096 7.7 against 7.0), or of 8192 weight rows.  Q4_K's pass is 6.5
+// us from the start.  Past those, Q4_K / Q5_K win from 2 rows (11008 x 4096: 11.9
+// against 13.8 us, 12.6 against 14.1), the rest from 3 (Q4_0 13.7 against 14.9; at
+// 2, 13.6 against 12.7), MXFP4 and the formats with two scales a block from 4
+// (NVFP4 18.3 against 17.0 at 3).  A quantized src1 is one launch either way.
+//
+// From 16 rows the other is the prefill GEMM, which takes one K loop of a 64 x
+// 128 tile whatever N is until the tiles fill the chip, while this kernel's time
+// grows with the weight rows times the token tiles; both grow with K.  The
+// limits are where the two lines measured at 4096 and 11008 x 4096, 16 .. 64
+// rows, cross (MXFP4, 64 rows: 20.7 against 33.0 us at 4096 rows, 41.0 against
+// 35.3 at 11008); at 512 .. 14336 values, 16 .. 64 rows and row counts up to
+// them no call was more than 3 % slower but for two, which have limits of their
+// own: MXFP4 past 3072 values, where a second round of workgroups is not worth
+// it (13000 x 11008, 32 rows: 65.3 against 58.1), and Q4_K at 17 .. 32 rows,
+// whose GEMM then has tiles of 32 x 64 (5632 x 512 7.0 against 6.4, 5120 x 2048
+// 9.7 against 9.1; 4096 x 2048 7.5 against 9.1, 5120 x 4096 equal).
+static bool small_wins(int fmt, size_t N, size_t K, size_t M, bool gemm, bool quantize) {
   static constexpr uint8_t kFrom[9] = {3, 4, 3, 4, 2, 4, 3, 4, 2};
   static constexpr uint16_t kLimit[9] = {21000, 14000, 20000, 17000, 27000, 28000, 21000, 18000, 8192};
   if (M < kFrom[fmt]) return false;
+  const size_t pass = M >= 3 && (fmt == 3 || fmt == 4 || fmt == 5) ? (size_t)16 << 20 : (size_t)28 << 20;
+  if (quantize && M <= 4 && fmt != 8 && M * K < 16384 && N < 8192 && M * N * K < pass) return false;
   if (M < 16 || !gemm) return true;
   if (M > kSmallBatchRows) return false;
-  // one token tile of 16 costs five eighths of one of 32; Q4_K's GEMM is 1.5
-  // times longer past 32 rows
+  size_t limit = kLimit[fmt];
+  if (fmt == 1 && K > 3072) limit = 12288;
+  if (fmt == 8 && M > 32) limit = limit * 3 / 2;  // its GEMM is 1.5 times longer past 32 rows
+  if (fmt == 8 && M > 16 && M <= 32 && K <= 2048) limit = 4096;
+  // one token tile of 16 costs five eighths of one of 32
   const size_t w = M <= 16 ? N * 5 / 8 : N * ((M + 31) / 32);
-  return w <= (fmt == 8 && M > 32 ? kLimit[fmt] * 3u / 2u : kLimit[fmt]);
+  return w <= limit;
 }
 
 static bool small_run(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
                       float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm, bool wide) {
-  if (!small_wins(fmt, N, M, gemm) || st.ldy < N || st.ldy >= ((size_t)1 << 38) ||
+  if (!small_wins(fmt, N, K, M, gemm, !wide) || st.ldy < N || st.ldy >= ((size_t)1 << 38) ||
       !small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, M, st)) return false;
   const FmtInfo f = fmt_info(fmt);
   const Args a{W, Xq, tab0, tab1, Y, (int)N, (int)K, (int)M, 1, (uint32_t)(N > 1 ? st.ldw : K / f.elems * f.rec),
@@ -930,7 +951,7 @@ void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab
 
 bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* tab0, const void* tab1,
                  float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm) {
-  if (X == nullptr || !aligned(X, 4) || !small_wins(fmt, N, M, gemm) || st.ldx < K || st.ldy < N ||
+  if (X == nullptr || !aligned(X, 4) || !small_wins(fmt, N, K, M, gemm, true) || st.ldx < K || st.ldy < N ||
       st.ldx >= ((size_t)1 << 38) || st.ldy >= ((size_t)1 << 38) || !small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, M, st))
     return false;
   switch (fmt) {
