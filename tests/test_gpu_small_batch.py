@@ -226,3 +226,29 @@ def test_any_bsums(hip, fmt, m):
 def test_waves_of_a_workgroup(hip, fmt, n, k, m):
     """Each choice of the waves that share K, on both sides of where it changes."""
     assert "small_mfma_gemm" in launched(hip, fmt, k, n, m)
+
+
+@pytest.mark.parametrize("fmt,n,k,experts,used,m,small", [
+    ("q4_k", 10240, 4096, 4, 1, 3, False), ("q4_k", 10240, 4096, 4, 1, 4, True),
+    ("q4_k", 10240, 4096, 4, 2, 2, False), ("q4_k", 10239, 4096, 4, 2, 2, True),
+    ("q4_k", 8192, 4096, 4, 1, 2, False), ("q4_k", 8192, 4096, 4, 1, 3, True),
+    ("q4_k", 4096, 8192, 4, 1, 2, False), ("q4_k", 4096, 8448, 4, 1, 2, True),
+    ("q4_k", 6144, 4096, 3, 1, 2, False), ("q4_k", 4096, 4096, 4, 1, 2, True),
+    ("nvfp4", 10240, 4096, 4, 1, 2, False), ("nvfp4", 10240, 4096, 4, 1, 3, True),
+    ("nvfp4", 10240, 4096, 4, 2, 2, True), ("q5_k", 10240, 4096, 4, 1, 2, True),
+])
+def test_pairs_that_share_little(hip, fmt, n, k, experts, used, m, small):
+    """Few pairs of large matrices stay on the pair GEMV (weights of zeros: which
+    kernel runs, and zeros out)."""
+    from weft_amd import _lib, ggml as G
+    w = hip.torch.zeros(experts * n * o.record_bytes(fmt, k), dtype=hip.torch.uint8, device=hip.dev)
+    x, y = hip.empty(4 * m * k), hip.empty(4 * m * used * n, fill=0xA5)
+    ids = hip.to_dev(np.array([[(t + s) % experts for s in range(used)] for t in range(m)], np.int32))
+    s0, s1 = G.tensor(TYPE[fmt], (k, n, experts), w.data_ptr()), G.tensor(G.F32, (k, 1, m), x.ptr)
+    it = G.tensor(G.I32, (used, m), ids.ptr)
+    work = hip.empty(G.mul_mat_id_work_size(s0, s1, it))
+    _lib.launch_log()
+    G.mul_mat_id(s0, s1, it, G.tensor(G.F32, (n, used, m), y.ptr), work.ptr, work.nbytes)
+    hip.torch.cuda.synchronize()
+    assert ("small_mfma_gemm_grouped" in _lib.launch_log()) == small
+    assert not y.numpy(np.float32).any()

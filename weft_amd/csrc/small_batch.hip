@@ -935,10 +935,31 @@ bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const i
   return small_run(fmt, W, Xq, tab0, tab1, Y, N, K, M, st, gemm, true);
 }
 
+// Whether MUL_MAT_ID's pair GEMV, one launch that reads an expert's weights once
+// for every pair of it, is the faster one: large matrices that it reads faster
+// than this kernel does, of which few pairs share an expert.  The first token's
+// pairs never do; `rest` of the others may.  Q4_K, whose GEMV keeps a row of up to
+// 4096 values in registers (one call, experts past the Infinity Cache): 14336 x
+// 4096, 2 pairs 14.8 us against 19.7 here, 16 experts of it, 2 a token, 2 / 4 / 6
+// tokens 44 / 46 / 67 against 47 / 49 / 68, 8 tokens 83 against 75; 6144 x 8192, 8
+// experts, 2 tokens 26.5 against 29.3; 4096 x 4096 equal from 2 pairs on.  NVFP4,
+// whose weights take this kernel longest, where a token has one expert: 11008 x
+// 4096, 2 / 3 pairs 21.3 / 30.6 against 25.6 / 34.2.  Of the other formats the
+// GEMV is at most as fast but for single shapes at 2 pairs.
+static bool pair_gemv_wins(int fmt, size_t N, size_t K, const PairArgs& pr, int n_pairs) {
+  const size_t values = N * K;
+  const int rest = n_pairs - pr.n_ids;
+  if (fmt == 5) return pr.n_ids == 1 && K > 2048 && values >= (size_t)40 << 20 && (rest == 1 || 8 * rest <= pr.n_as);
+  if (fmt != 8 || K > 8192) return false;
+  if (K > 2048 && K <= 4096 && values >= (size_t)40 << 20) return rest <= 10 && 2 * rest <= pr.n_as;
+  if (values >= (size_t)32 << 20) return rest <= 3 && 4 * rest <= pr.n_as;
+  return n_pairs == 2 && values >= (size_t)24 << 20;
+}
+
 bool small_pairs_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1,
                     const float* Y, size_t N, size_t K, const RowStrides& st, const PairArgs& pr, int n_pairs,
                     size_t x_rows) {
-  return n_pairs >= 2 && n_pairs <= 64 && pr.w_es % (long long)fmt_info(fmt).w_align == 0 &&
+  return n_pairs >= 2 && n_pairs <= 64 && !pair_gemv_wins(fmt, N, K, pr, n_pairs) && pr.w_es % (long long)fmt_info(fmt).w_align == 0 &&
          small_ok(fmt, W, Xq, tab0, tab1, Y, N, K, x_rows, st);
 }
 void small_pairs(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t* tab0, const void* tab1, float* Y,
