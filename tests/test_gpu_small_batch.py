@@ -252,3 +252,10 @@ def test_pairs_that_share_little(hip, fmt, n, k, experts, used, m, small):
     hip.torch.cuda.synchronize()
     assert ("small_mfma_gemm_grouped" in _lib.launch_log()) == small
     assert not y.numpy(np.float32).any()
+
+
+@pytest.mark.parametrize("fmt,k,pad", [("q4_k", 512, 2), ("q5_k", 512, 2), ("q6_k", 512, 1), ("iq2_xxs", 768, 0),
+                                       ("iq2_xs", 768, 0)])
+def test_many_q8k_rows_no_gemm_takes(hip, fmt, k, pad):
+    # a Q8_K src1 on weights off 4-byte alignment (Q6_K: off 2), an odd superblock count
+    assert launched(hip, fmt, k, 75, 70, pad_w=pad, prequant=True) == ["small_mfma_gemm"]

@@ -342,7 +342,8 @@ hipError_t mul_mat(const weft_ggml_tensor* s0, const weft_ggml_tensor* s1, const
       } else if (small_batch_quantized(gemv_format(s0->type), W, src1, tables0(tab, s0->type), tables1(tab, s0->type), Y,
                                        n, k, m, st, vd->size == kQ8_KBytes)) {
         // done: a few rows of an activation that is already quantized, any
-        // number of them as Q8_0 / Q8_1 (those formats' GEMMs quantize X)
+        // number of them as Q8_0 / Q8_1 (those formats' GEMMs quantize X; the
+        // Q8_K ones below come back to it for weights they do not take)
       } else {
         switch (s0->type) {
           case WEFT_GGML_TYPE_Q4_0: decode_quantized(0, W, src1, nullptr, nullptr, Y, n, k, m, st); break;

@@ -517,16 +517,22 @@ void mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t*
 
 void mul_mat_iq2_xs_quantized(const uint8_t* W, const uint8_t* Xq, const int8_t* grid, const int8_t* signs,
                               float* Y, size_t N, size_t K, size_t M, const RowStrides& st) {
-  if (!gemm_iq2_ok<true>(W, Xq, Y, grid, signs, N, K, M, st))
-    return decode_quantized(7, W, Xq, grid, signs, Y, N, K, M, st);
+  if (!gemm_iq2_ok<true>(W, Xq, Y, grid, signs, N, K, M, st)) {
+    if (!small_batch_quantized(7, W, Xq, grid, signs, Y, N, K, M, st, false))
+      decode_quantized(7, W, Xq, grid, signs, Y, N, K, M, st);
+    return;
+  }
   gemm_iq2<true>(W, Xq, grid, signs, Y, N, K, M, st);
 }
 
 void mul_mat_iq2_xxs_quantized(const uint8_t* W, const uint8_t* Xq, const int8_t* grid,
                                const int8_t* signs, float* Y, size_t N, size_t K, size_t M,
                                const RowStrides& st) {
-  if (!gemm_iq2_ok(W, Xq, Y, grid, signs, N, K, M, st))
-    return decode_quantized(2, W, Xq, grid, signs, Y, N, K, M, st);
+  if (!gemm_iq2_ok(W, Xq, Y, grid, signs, N, K, M, st)) {
+    if (!small_batch_quantized(2, W, Xq, grid, signs, Y, N, K, M, st, false))
+      decode_quantized(2, W, Xq, grid, signs, Y, N, K, M, st);
+    return;
+  }
   gemm_iq2(W, Xq, grid, signs, Y, N, K, M, st);
 }
 

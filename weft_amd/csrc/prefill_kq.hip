@@ -557,15 +557,21 @@ void mul_mat_q5k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t
 
 void mul_mat_q6k_quantized(const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
                            const RowStrides& st) {
-  if (!gemm_kq_ok<KQ::Q6_K>(W, Xq, Y, N, K, M, st))
-    return decode_quantized(3, W, Xq, nullptr, nullptr, Y, N, K, M, st);
+  if (!gemm_kq_ok<KQ::Q6_K>(W, Xq, Y, N, K, M, st)) {
+    if (!small_batch_quantized(3, W, Xq, nullptr, nullptr, Y, N, K, M, st, false))
+      decode_quantized(3, W, Xq, nullptr, nullptr, Y, N, K, M, st);
+    return;
+  }
   gemm_kq<KQ::Q6_K>(W, Xq, Y, N, K, M, st);
 }
 
 void mul_mat_q5k_quantized(const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
                            const RowStrides& st) {
-  if (!gemm_kq_ok<KQ::Q5_K>(W, Xq, Y, N, K, M, st))
-    return decode_quantized(4, W, Xq, nullptr, nullptr, Y, N, K, M, st);
+  if (!gemm_kq_ok<KQ::Q5_K>(W, Xq, Y, N, K, M, st)) {
+    if (!small_batch_quantized(4, W, Xq, nullptr, nullptr, Y, N, K, M, st, false))
+      decode_quantized(4, W, Xq, nullptr, nullptr, Y, N, K, M, st);
+    return;
+  }
   gemm_kq<KQ::Q5_K>(W, Xq, Y, N, K, M, st);
 }
 

@@ -693,7 +693,7 @@ void mul_mat_q4k_quantized(const uint8_t* W, const uint8_t* Xq, float* Y, size_t
   if (N == 0 || M == 0 || K == 0) return;
   if ((M >= 16 || !q4k_gemv_fits(K)) && args_ok(W, Xq, Y, N, K, M, st) && gemm_q4k_ok(W, N, K, M, st))
     gemm_q4k(W, Xq, Y, N, K, M, st);
-  else
+  else if (!small_batch_quantized(8, W, Xq, nullptr, nullptr, Y, N, K, M, st, false))
     decode_q4k_quantized(W, Xq, Y, N, K, M, st);
 }
 
