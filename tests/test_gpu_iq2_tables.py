@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from tests.test_gpu_parity import SENTINEL, acts, assert_close
+from tests.test_gpu_parity import GEMM, SENTINEL, acts, assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -77,13 +77,14 @@ def run(hip, symbol, fmt, grid, signs, n, k, m, seed=83):
     ("decode", 1000, 4096, 1, "iq2_gemv_m1_kernel"),  # batch 1, K <= 4096
     ("decode", 300, 1024, 3, "staged_gemv_kernel"),   # 1 < M < 16
     ("decode", 64, 5120, 1, "staged_gemv_kernel"),    # K > 4096
-    ("prefill", 200, 1024, 64, "mfma_gemm"),          # the MFMA GEMM
+    ("prefill", 200, 1024, 64, "small_mfma_gemm"),    # the small-batch kernel
+    ("prefill", 200, 1024, 70, GEMM),                 # the MFMA GEMM
 ])
 def test_caller_tables(hip, fmt, case, path, n, k, m, kernel):
     grid, signs = table_cases(fmt)[case]
     symbol = (DECODE if path == "decode" else PREFILL)[fmt]
     launched = run(hip, symbol, fmt, grid, signs, n, k, m)
-    assert any(kernel in name for name in launched), launched
+    assert (kernel[fmt] if kernel is GEMM else kernel) in launched, launched
 
 
 @pytest.mark.parametrize("fmt", ["iq2_xxs", "iq2_xs"])
@@ -103,5 +104,6 @@ def test_ggml_tables_keep_the_mask_path_result(hip, fmt):
     """GGML's own tables give the same result as the oracle restated for
     caller tables, on every path (they take the mask path)."""
     grid, signs = ggml_tables(fmt)
-    for symbol, n, k, m in ((DECODE[fmt], 500, 4096, 1), (PREFILL[fmt], 200, 1024, 64)):
+    for symbol, n, k, m in ((DECODE[fmt], 500, 4096, 1), (PREFILL[fmt], 200, 1024, 64),
+                            (PREFILL[fmt], 200, 1024, 70)):
         run(hip, symbol, fmt, grid, signs, n, k, m)

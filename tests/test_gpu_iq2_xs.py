@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from tests.test_gpu_parity import SENTINEL, acts, assert_close, check_mul_mat, run_mul_mat
+from tests.test_gpu_parity import SENTINEL, acts, assert_close, assert_prefill_kernel, check_mul_mat, run_mul_mat
 
 pytestmark = pytest.mark.gpu
 
@@ -119,16 +119,19 @@ def extreme_weights(n, k, seed=23):
     return np.ascontiguousarray(w.reshape(n, -1))
 
 
-def test_prefill_iq2_xs_extreme_records(hip):
-    """The MFMA GEMM (per-16 scales, sign masks from LDS, the dx dw factor
+@pytest.mark.parametrize("m", [48, 70])
+def test_prefill_iq2_xs_extreme_records(hip, m):
+    """The small-batch kernel and the MFMA GEMM (per-16 scales, sign masks from LDS, the dx dw factor
     from a bf16 outer-product MFMA) on corner records, against activations
     with an all-zero Q8_K block and an all-zero token."""
-    n, k, m = 160, 2048, 48
+    n, k = 160, 2048
     w = extreme_weights(n, k)
     x = acts(m, k, seed=9).copy()
     x[4, 256:512] = 0.0
     x[7] = 0.0
+    hip._lib.launch_log()
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_iq2_xs", "iq2_xs", n, k, m, w=w, x=x)
+    assert_prefill_kernel(hip, "iq2_xs", m)
     check_mul_mat("iq2_xs", w, x, xq, y, n, k, m)
 
 

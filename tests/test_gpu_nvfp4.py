@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from tests.test_gpu_parity import SENTINEL, acts, assert_close, check_mul_mat, run_mul_mat, weights
+from tests.test_gpu_parity import SENTINEL, acts, assert_close, assert_prefill_kernel, check_mul_mat, run_mul_mat, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -97,15 +97,18 @@ def test_prefill_nvfp4(hip, n, k, m):
     check_mul_mat("nvfp4", w, x, xq, y, n, k, m)
 
 
-def test_prefill_nvfp4_extreme_records(hip):
-    """The MFMA GEMM on rows that cycle through all 256 UE4M3 scale bytes
+@pytest.mark.parametrize("m", [40, 70])
+def test_prefill_nvfp4_extreme_records(hip, m):
+    """The small-batch kernel and the MFMA GEMM on rows that cycle through all 256 UE4M3 scale bytes
     (0x00 and 0x7F read as zero, subnormals, 448) and every code, against
     activations with an all-zero Q8_0 block and an all-zero token."""
-    n, k, m = 128, 4096, 40
+    n, k = 128, 4096
     recs = extreme_records()                  # 64 records = one row of K = 4096
     w = np.stack([np.roll(recs, 5 * r, axis=0) for r in range(n)]).reshape(n, -1)
     x = acts(m, k, seed=9).copy()
     x[4, 64:96] = 0.0
     x[7] = 0.0
+    hip._lib.launch_log()
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_nvfp4", "nvfp4", n, k, m, w=w, x=x)
+    assert_prefill_kernel(hip, "nvfp4", m)
     check_mul_mat("nvfp4", w, x, xq, y, n, k, m)

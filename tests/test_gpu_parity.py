@@ -51,6 +51,21 @@ def tables(hip, fmt):
     return []
 
 
+# what a prefill call launches after its quantization: the small-batch kernel up
+# to 64 rows (fewer for many weight rows), the format's GEMM past that
+GEMM = {"q4_0": "q80_mfma_gemm", "q4_1": "q80_mfma_gemm", "mxfp4": "mxfp4_gemm", "nvfp4": "nvfp4_mfma_gemm",
+        "q4_k": "q4k_mfma_gemm", "q5_k": "q5k_mfma_gemm", "q6_k": "q6k_mfma_gemm",
+        "iq2_xxs": "iq2_mfma_gemm", "iq2_xs": "iq2xs_mfma_gemm"}
+
+
+def assert_prefill_kernel(hip, fmt, m):
+    """The launches since the log was last read hold the kernel meant for m rows
+    (Q4_K's GEMM is named with its tile)."""
+    names = {name.split("_mfma_gemm_")[0] + "_mfma_gemm" if name.startswith("q4k_mfma_gemm_") else name
+             for name in hip._lib.launch_log()}
+    assert ("small_mfma_gemm" if m <= 64 else GEMM[fmt]) in names, names
+
+
 def assert_close(y, e, a, what):
     ok = o.within_tolerance(y, e, a)
     if not ok.all():
@@ -509,28 +524,32 @@ def test_decode_iq2_xxs_batch1(hip, n, k):
     check_mul_mat("iq2_xxs", w, x, xq, y, n, k, 1)
 
 
+@pytest.mark.parametrize("m", [64, 70])
 @pytest.mark.parametrize("fmt,make", [("q4_k", crafted_q4_k), ("q4_0", crafted_q4_0),
                                       ("iq2_xxs", crafted_iq2_xxs)])
-def test_prefill_crafted_records(hip, fmt, make):
-    """The MFMA prefill GEMMs on records no quantizer emits: d / dmin zero,
+def test_prefill_crafted_records(hip, fmt, make, m):
+    """The small-batch kernel and the MFMA prefill GEMMs on records no quantizer emits: d / dmin zero,
     negative zero, subnormal, the smallest normal and +-65504; Q4_K sub-blocks
     with sc = m = 63 and all-15 nibbles; Q4_0 blocks of q - 8 = -8; IQ2_XXS
     groups with scale 15 and 0; activations with all-zero Q8_K blocks and
     rows, a dominant element and a negative maximum."""
     rng = np.random.default_rng(77)
-    n, k, m = 256, 1024, 64
+    n, k = 256, 1024
     w = make(n, k, rng)
     x = crafted_acts_q8k(m, k, rng)
     print(f"crafted prefill {fmt}", flush=True)
+    hip._lib.launch_log()
     w, x, xq, y = run_mul_mat(hip, MM_PREFILL[fmt], fmt, n, k, m, w=w, x=x)
+    assert_prefill_kernel(hip, fmt, m)
     check_mul_mat(fmt, w, x, xq, y, n, k, m)
 
 
-def test_prefill_mxfp4_crafted_scales(hip):
-    """MXFP4 prefill on the block-scaled MFMA with every nibble and a wide
+@pytest.mark.parametrize("m", [64, 70])
+def test_prefill_mxfp4_crafted_scales(hip, m):
+    """MXFP4 prefill (the small-batch kernel, the block-scaled MFMA) with every nibble and a wide
     spread of E8M0 exponents (2..200, whole rows at both ends), not just the
     few a quantizer emits; products stay inside fp32's range."""
-    n, k, m = 256, 1024, 64
+    n, k = 256, 1024
     rng = np.random.default_rng(21)
     rec = rng.integers(0, 256, size=(n, k // 32, 17), dtype=np.uint8)
     rec[:, :, 0] = rng.integers(2, 201, size=(n, k // 32), dtype=np.uint8)
@@ -540,24 +559,30 @@ def test_prefill_mxfp4_crafted_scales(hip):
     x = acts(m, k)
     xq = hip.empty(o.record_bytes("q8_0", k) * m, fill=SENTINEL)
     y = hip.empty(4 * m * n, fill=SENTINEL)
+    hip._lib.launch_log()
     hip.call("production_mul_mat_mxfp4", hip.to_dev(w), hip.to_dev(x), xq, hip.codebook, hip.scale, y,
              n, k, m)
+    assert_prefill_kernel(hip, "mxfp4", m)
     check_mul_mat("mxfp4", w, x, xq.numpy(np.uint8).reshape(m, -1), y.numpy(np.float32).reshape(m, n),
                   n, k, m)
 
 
-@pytest.mark.parametrize("symbol,m", [("production_mul_mat_mxfp4", 64), ("production_mul_mat_mxfp4_decode", 1)])
+@pytest.mark.parametrize("symbol,m", [("production_mul_mat_mxfp4", 64), ("production_mul_mat_mxfp4", 70),
+                                      ("production_mul_mat_mxfp4_decode", 1)])
 def test_mxfp4_caller_tables_are_used(hip, symbol, m):
     """A scale table that is not GGML's (every entry doubled) is honoured:
-    the prefill takes the table-driven int8-MFMA GEMM and the result is
-    exactly twice GGML's."""
+    64 rows take the small-batch kernel, 70 the GEMM's table-driven int8-MFMA
+    body, and the result is exactly twice GGML's."""
     n, k = 256, 1024
     w, x = weights("mxfp4", n, k), acts(m, k)
     with np.errstate(over="ignore"):  # entry 255 (2^127) doubles to inf
         scale2 = hip.to_dev(2.0 * o.e8m0_half_table())
     xq = hip.empty(o.record_bytes("q8_0", k) * m, fill=SENTINEL)
     y = hip.empty(4 * m * n, fill=SENTINEL)
+    hip._lib.launch_log()
     hip.call(symbol, hip.to_dev(w), hip.to_dev(x), xq, hip.codebook, scale2, y, n, k, m)
+    if m > 1:
+        assert_prefill_kernel(hip, "mxfp4", m)
     want_xq = np.full((m, o.record_bytes("q8_0", k)), SENTINEL, np.uint8)
     o.quantize("q8_0", x, out=want_xq)
     np.testing.assert_array_equal(xq.numpy(np.uint8).reshape(m, -1), want_xq)
@@ -567,19 +592,24 @@ def test_mxfp4_caller_tables_are_used(hip, symbol, m):
 
 @pytest.mark.parametrize("fmt,symbol,m", [
     ("mxfp4", "production_mul_mat_mxfp4_decode", 1), ("mxfp4", "production_mul_mat_mxfp4", 64),
-    ("nvfp4", "production_mul_mat_nvfp4_decode", 1), ("nvfp4", "production_mul_mat_nvfp4", 64)])
+    ("mxfp4", "production_mul_mat_mxfp4", 70),
+    ("nvfp4", "production_mul_mat_nvfp4_decode", 1), ("nvfp4", "production_mul_mat_nvfp4", 64),
+    ("nvfp4", "production_mul_mat_nvfp4", 70)])
 def test_fp4_caller_codebook_is_used(hip, fmt, symbol, m):
     """A codebook that is not GGML's (kvalues_mxfp4 negated) is honoured:
     the batch-1 kernels look it up with v_perm instead of converting the
-    nibbles as E2M1 codes, the prefill takes its table-driven body, and the
-    result is exactly minus GGML's."""
+    nibbles as E2M1 codes, 64 rows take the small-batch kernel, 70 the GEMM's
+    table-driven body, and the result is exactly minus GGML's."""
     n, k = 256, 1024
     w, x = weights(fmt, n, k), acts(m, k)
     neg = hip.to_dev((-o.kvalues_mxfp4().astype(np.int16)).astype(np.int8))
     tab = hip.scale if fmt == "mxfp4" else hip.ue4m3
     xq = hip.empty(o.record_bytes("q8_0", k) * m, fill=SENTINEL)
     y = hip.empty(4 * m * n, fill=SENTINEL)
+    hip._lib.launch_log()
     hip.call(symbol, hip.to_dev(w), hip.to_dev(x), xq, neg, tab, y, n, k, m)
+    if m > 1:
+        assert_prefill_kernel(hip, fmt, m)
     want_xq = np.full((m, o.record_bytes("q8_0", k)), SENTINEL, np.uint8)
     o.quantize("q8_0", x, out=want_xq)
     np.testing.assert_array_equal(xq.numpy(np.uint8).reshape(m, -1), want_xq)

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from tests.test_gpu_parity import (FP16_EDGES, SENTINEL, acts, assert_close, check_mul_mat,
+from tests.test_gpu_parity import (FP16_EDGES, SENTINEL, acts, assert_close, assert_prefill_kernel, check_mul_mat,
                                    crafted_acts_q8k, edge_rows, run_mul_mat, weights)
 
 pytestmark = pytest.mark.gpu
@@ -99,12 +99,15 @@ def test_prefill_q4_1(hip, n, k, m):
     check_mul_mat("q4_1", w, x, xq, y, n, k, m)
 
 
-def test_prefill_q4_1_crafted_records(hip):
+@pytest.mark.parametrize("m", [64, 70])
+def test_prefill_q4_1_crafted_records(hip, m):
     rng = np.random.default_rng(79)
-    n, k, m = 256, 1024, 64
+    n, k = 256, 1024
     w = crafted_q4_1(n, k, rng)
     x = crafted_acts_q8k(m, k, rng)
+    hip._lib.launch_log()
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q4_1", "q4_1", n, k, m, w=w, x=x)
+    assert_prefill_kernel(hip, "q4_1", m)
     check_mul_mat("q4_1", w, x, xq, y, n, k, m)
 
 

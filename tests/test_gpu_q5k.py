@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as o
-from tests.test_gpu_parity import SENTINEL, acts, assert_close, check_mul_mat, run_mul_mat, weights
+from tests.test_gpu_parity import SENTINEL, acts, assert_close, assert_prefill_kernel, check_mul_mat, run_mul_mat, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -101,11 +101,12 @@ def test_prefill_q5_k(hip, n, k, m):
     check_mul_mat("q5_k", w, x, xq, y, n, k, m)
 
 
-def test_prefill_q5_k_extreme_records(hip):
-    """The MFMA GEMM on whole rows of 0 and 31 codes, scales and mins at 63,
+@pytest.mark.parametrize("m", [48, 70])
+def test_prefill_q5_k_extreme_records(hip, m):
+    """The small-batch kernel and the MFMA GEMM on whole rows of 0 and 31 codes, scales and mins at 63,
     d = 0 with dmin kept, against activations with an all-zero Q8_K block and
     an all-zero token."""
-    n, k, m = 160, 2048, 48
+    n, k = 160, 2048
     w = extreme_records(n * k // 256).reshape(n, k // 256, 176)
     w[5, :, 16:176] = 0x00
     w[9, :, 16:176] = 0xFF
@@ -116,5 +117,7 @@ def test_prefill_q5_k_extreme_records(hip):
     x = acts(m, k, seed=9).copy()
     x[4, 256:512] = 0.0
     x[7] = 0.0
+    hip._lib.launch_log()
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q5_k", "q5_k", n, k, m, w=w, x=x)
+    assert_prefill_kernel(hip, "q5_k", m)
     check_mul_mat("q5_k", w, x, xq, y, n, k, m)
