@@ -50,7 +50,8 @@ void *weft_hip_get_stream(void);
  * counterpart in the generated C, where they are compile-time constants):
  * "NC" = weight rows per workgroup and "MR" = activation rows per pass
  * (1..4) of the GEMV kernels; for the Q4_K prefill GEMM (M >= 16 of
- * production_mul_mat_q4_k_staged / production_mul_mat_q4_k) "NC" = weight
+ * production_mul_mat_q4_k_staged / production_mul_mat_q4_k; a call with a binding
+ * set does not run the small-batch kernel) "NC" = weight
  * rows per tile (<= 64: 64, else 128) and "MC" = activation rows per tile
  * (<= 32: 32, else 64); 0 unsets.  Returns 1 when the name has a launch
  * knob here, 0 otherwise (KC, NR and the other MFMA GEMMs' fixed 64 x 128

@@ -70,7 +70,7 @@ def test_vec_dot_nvfp4_extreme_records(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 1), (11008, 4096, 1), (4096, 14336, 1), (300, 768, 3),
                                    (65, 1024, 5), (1, 64, 1), (17, 1024, 1), (5000, 2048, 1)])
 def test_decode_nvfp4(hip, n, k, m):
-    """M = 1 with K <= 4096 a multiple of 64 runs the batch-1 kernel (records
+    """M = 1 with K <= 16384 a multiple of 64 runs the batch-1 kernel (records
     in VGPRs), every other shape the staged GEMV."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_nvfp4_decode", "nvfp4", n, k, m)
     check_mul_mat("nvfp4", w, x, xq, y, n, k, m)
@@ -91,8 +91,9 @@ def test_decode_nvfp4_batch1_extreme_records(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 512), (512, 4096, 64), (144, 768, 70), (129, 256, 17),
                                    (300, 320, 40), (64, 512, 15)])
 def test_prefill_nvfp4(hip, n, k, m):
-    """M >= 16 with K a multiple of 256 runs the int8-MFMA GEMM (ragged
-    weight and token tiles included); K = 320 and M = 15 take the GEMV."""
+    """More than 64 rows with K a multiple of 256 run the int8-MFMA GEMM (ragged
+    weight and token tiles included), 15 to 64 here the small-batch kernel;
+    K = 320 takes the GEMV."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_nvfp4", "nvfp4", n, k, m)
     check_mul_mat("nvfp4", w, x, xq, y, n, k, m)
 

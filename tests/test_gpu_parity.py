@@ -261,11 +261,11 @@ def test_decode_small_shapes(hip, fmt, n, k, m):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q4_k", "iq2_xxs", "mxfp4"])
-@pytest.mark.parametrize("m", [1, 3, 64])
+@pytest.mark.parametrize("m", [1, 3, 64, 70])
 def test_long_rows(hip, fmt, m):
-    """K = 65536: the batch-1 and small-batch GEMVs stage the whole quantized
-    activation row in LDS (about 72 KB), the prefill GEMMs stream it by
-    superblock pairs."""
+    """K = 65536: the GEMVs stage the whole quantized activation row in LDS
+    (about 72 KB), the small-batch kernel (64 rows) and the prefill GEMMs (70)
+    stream it."""
     n, k = 96, 65536
     w, x, xq, y = run_mul_mat(hip, MM_PREFILL[fmt] if m >= 16 else MM_DECODE[fmt], fmt, n, k, m)
     check_mul_mat(fmt, w, x, xq, y, n, k, m)
@@ -290,8 +290,8 @@ def launch_log(hip):
 def test_long_row_small_batch_takes_the_gemm(hip, fmt, m):
     """K = 2^18 (a quantized activation row of ~300 KB, past a workgroup's
     LDS) below 16 activation rows: the mul_mat entry points run the
-    format's prefill GEMM, which streams K, instead of the GEMVs that keep
-    the row in LDS; every output against the oracle."""
+    format's prefill GEMM or the small-batch kernel, which stream K, instead of
+    the GEMVs that keep the row in LDS; every output against the oracle."""
     n, k = 8, 1 << 18
     x = o.seeded_normal(31, (m, k))
     w = (o.random_records(fmt, n, k, seed=32) if fmt.startswith("iq2")
@@ -399,12 +399,14 @@ def test_prefill_entry_points(hip, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q4_0", "mxfp4", "iq2_xxs"])
-@pytest.mark.parametrize("n,k,m", [(300, 512, 37), (129, 768, 16), (128, 256, 65), (200, 1536, 70)])
+@pytest.mark.parametrize("n,k,m", [(300, 512, 37), (129, 768, 16), (128, 256, 65), (200, 1536, 70),
+                                   (129, 768, 70)])
 def test_prefill_ragged_tiles(hip, fmt, n, k, m):
     # shapes that leave partial 64 x 128 MFMA tiles on both axes, an odd
     # number of 256-value stages (K = 768) for the stage-parity waves, and an
-    # odd number of stage pairs (K = 1536) for the two LDS ring slots; IQ2_XXS
-    # at K = 768 / 256 takes the GEMV path (its GEMM stages superblock pairs)
+    # odd number of stage pairs (K = 1536) for the two LDS ring slots; up to 64
+    # rows, and IQ2_XXS at K = 768 / 256 (its GEMM stages superblock pairs), the
+    # small-batch kernel
     w, x, xq, y = run_mul_mat(hip, MM_PREFILL[fmt], fmt, n, k, m)
     check_mul_mat(fmt, w, x, xq, y, n, k, m)
 
@@ -412,7 +414,7 @@ def test_prefill_ragged_tiles(hip, fmt, n, k, m):
 @pytest.mark.parametrize("fmt", ["q4_0", "mxfp4", "iq2_xxs"])
 def test_prefill_misaligned_weights_fall_back(hip, fmt):
     # W at a 2-byte offset is valid for these records but not for the MFMA
-    # path's 4-byte direct loads: the call must take the GEMV path and agree
+    # path's 4-byte direct loads: the call must take another kernel and agree
     n, k, m = 96, 512, 20
     w, x = weights(fmt, n, k), acts(m, k)
     act = o.ACT_OF[fmt]

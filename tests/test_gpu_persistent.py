@@ -7,8 +7,9 @@ Bars (declared before any run): the packed weight is byte-for-byte the
 oracle's 16-row interleave; Xq is bit-exact Q8_K of X; Y is within the fp64
 re-accumulation tolerance (|y - E| <= 1e-4 |E| + 4e-6 A) of the row-major
 records the packed bytes came from.  For M >= 16 the GEMM reads the same
-bytes in the same order as production_mul_mat_q4_k_staged, so the two
-outputs must be bit-identical.
+bytes in the same order as the row-major GEMM, which
+production_mul_mat_q4_k_staged runs past 64 rows, so the two outputs must be
+bit-identical there.
 """
 from __future__ import annotations
 

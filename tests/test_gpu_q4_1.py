@@ -75,7 +75,7 @@ def test_vec_dot_q4_1(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 1), (11008, 4096, 1), (4096, 14336, 1), (300, 768, 3),
                                    (65, 1024, 5), (1, 32, 1), (1, 64, 1), (17, 1024, 1), (5000, 2048, 1)])
 def test_decode_q4_1(hip, n, k, m):
-    """M = 1 with K <= 4096 a multiple of 64 runs the batch-1 kernel (records
+    """M = 1 with K <= 16384 a multiple of 64 runs the batch-1 kernel (records
     in VGPRs), every other shape the staged GEMV."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q4_1_decode", "q4_1", n, k, m)
     check_mul_mat("q4_1", w, x, xq, y, n, k, m)
@@ -92,9 +92,10 @@ def test_decode_q4_1_batch1_crafted_records(hip):
 
 
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 512), (300, 512, 37), (129, 768, 16), (200, 1536, 70),
-                                   (64, 4096, 8)])
+                                   (64, 4096, 8), (129, 768, 66)])
 def test_prefill_q4_1(hip, n, k, m):
-    """M >= 16 and K % 256 == 0 run the MFMA GEMM; (64, 4096, 8) the GEMV."""
+    """More than 64 rows and K % 256 == 0 run the MFMA GEMM, fewer here the
+    small-batch kernel."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q4_1", "q4_1", n, k, m)
     check_mul_mat("q4_1", w, x, xq, y, n, k, m)
 

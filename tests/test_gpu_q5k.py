@@ -70,7 +70,7 @@ def test_vec_dot_q5_k_extreme_records(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 1), (11008, 4096, 1), (4096, 14336, 1), (300, 768, 3),
                                    (65, 1024, 5), (1, 256, 1), (17, 1024, 1), (5000, 2048, 1), (33, 768, 1)])
 def test_decode_q5_k(hip, n, k, m):
-    """M = 1 with K <= 4096 runs the batch-1 kernel (records in VGPRs),
+    """M = 1 with K <= 16384 runs the batch-1 kernel (records in VGPRs),
     every other shape the staged GEMV."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q5_k_decode", "q5_k", n, k, m)
     check_mul_mat("q5_k", w, x, xq, y, n, k, m)
@@ -93,10 +93,10 @@ def test_decode_q5_k_batch1_extreme_records(hip):
 
 
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 512), (512, 4096, 64), (144, 1024, 70), (300, 768, 17),
-                                   (129, 256, 40), (64, 512, 15)])
+                                   (129, 256, 40), (64, 512, 15), (300, 768, 66), (129, 256, 65)])
 def test_prefill_q5_k(hip, n, k, m):
-    """M >= 16 runs the int8-MFMA GEMM (odd superblock counts, ragged weight
-    and token tiles included); M = 15 takes the GEMV."""
+    """More than 64 rows run the int8-MFMA GEMM (odd superblock counts, ragged
+    weight and token tiles included), 15 to 64 here the small-batch kernel."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q5_k", "q5_k", n, k, m)
     check_mul_mat("q5_k", w, x, xq, y, n, k, m)
 

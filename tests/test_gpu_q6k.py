@@ -62,7 +62,7 @@ def test_vec_dot_q6_k_extreme_records(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 1), (11008, 4096, 1), (4096, 14336, 1), (300, 768, 3),
                                    (65, 1024, 5), (1, 256, 1), (1, 512, 1), (17, 1024, 1), (5000, 2048, 1)])
 def test_decode_q6_k(hip, n, k, m):
-    """M = 1 with K <= 4096 a multiple of 512 runs the batch-1 kernel
+    """M = 1 with K <= 16384 runs the batch-1 kernel
     (records in VGPRs, odd superblocks at a 2-byte offset), every other
     shape the staged GEMV."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q6_k_decode", "q6_k", n, k, m)
@@ -91,8 +91,8 @@ def test_decode_q6_k_batch1_extreme_records(hip):
 @pytest.mark.parametrize("n,k,m", [(4096, 4096, 512), (512, 4096, 64), (144, 1024, 70), (129, 2048, 17),
                                    (300, 768, 40), (64, 512, 15)])
 def test_prefill_q6_k(hip, n, k, m):
-    """M >= 16 with K a multiple of 512 runs the int8-MFMA GEMM (ragged
-    weight and token tiles included); K = 768 and M = 15 take the GEMV."""
+    """More than 64 rows run the int8-MFMA GEMM (ragged weight and token tiles
+    included), 15 to 64 here the small-batch kernel."""
     w, x, xq, y = run_mul_mat(hip, "production_mul_mat_q6_k", "q6_k", n, k, m)
     check_mul_mat("q6_k", w, x, xq, y, n, k, m)
 

@@ -948,7 +948,7 @@ void production_mul_mat_q6_k_decode(const uint8_t* W, const float* X, uint8_t* X
   weft::decode_q6_k(W, X, Xq, Y, N, K, M, weft::packed(K / 256 * weft::kQ6_KBytes, K, N));
 }
 
-// Q6_K mul_mat: the int8-MFMA GEMM for prefill shapes, the GEMV otherwise
+// Q6_K mul_mat: the small-batch kernel, the int8-MFMA GEMM or the GEMV by rows (kernels.h)
 void production_mul_mat_q6_k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N,
                              size_t K, size_t M) {
   if (X == nullptr || Xq == nullptr) return weft::set_error(hipErrorInvalidValue);
@@ -963,7 +963,7 @@ void production_mul_mat_nvfp4_decode(const uint8_t* W, const float* X, uint8_t* 
                      weft::packed(K / 64 * weft::kNvfp4Bytes, K, N));
 }
 
-// NVFP4 mul_mat: the int8-MFMA GEMM for prefill shapes, the GEMV otherwise
+// NVFP4 mul_mat: the small-batch kernel, the int8-MFMA GEMM or the GEMV by rows (kernels.h)
 void production_mul_mat_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                               const float* scale, float* Y, size_t N, size_t K, size_t M) {
   if (X == nullptr || Xq == nullptr) return weft::set_error(hipErrorInvalidValue);
@@ -983,7 +983,7 @@ void production_mul_mat_q5_k_decode(const uint8_t* W, const float* X, uint8_t* X
   weft::decode_q5_k(W, X, Xq, Y, N, K, M, weft::packed(K / 256 * weft::kQ5_KBytes, K, N));
 }
 
-// Q5_K mul_mat: the int8-MFMA GEMM for prefill shapes, the GEMV otherwise
+// Q5_K mul_mat: the small-batch kernel, the int8-MFMA GEMM or the GEMV by rows (kernels.h)
 void production_mul_mat_q5_k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N,
                              size_t K, size_t M) {
   if (X == nullptr || Xq == nullptr) return weft::set_error(hipErrorInvalidValue);

@@ -59,7 +59,8 @@ bool decode_rec_m1(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const
 bool decode_q5k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st);
 // Batch-1 Q6_K GEMV with the records in VGPRs (decode_q6k.hip); false when
-// the call does not suit it (K > 4 * 4096, unaligned).
+// the call does not suit it (K > 4 * 4096, unaligned, many rows of three or
+// four whole steps).
 bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                    const RowStrides& st);
 // Batch-1 IQ2_XXS / IQ2_XS (xs) GEMV with the records in VGPRs (decode_iq2.hip);
@@ -154,7 +155,10 @@ void decode_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t
 void decode_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid,
                    const int8_t* signs, float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
 
-// Q4_K mul_mat for any M: int8-MFMA GEMM for prefill shapes, GEMV otherwise.
+// mul_mat for any M, this format's and the ones below: the small-batch kernel
+// for 2 .. 64 rows where it is the faster one (small_batch, below), the int8-MFMA
+// GEMM for prefill shapes, the small-batch kernel again for more rows of weights
+// that the GEMM does not take, the GEMV otherwise.  Q4_K:
 void mul_mat_q4k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                  size_t M, const RowStrides& st);
 // the same over an already quantized Q8_K activation
@@ -172,20 +176,20 @@ size_t q4k_i16_packed_size(size_t M, size_t K);
 void q4k_i16_pack(const uint8_t* source, uint8_t* target, size_t M, size_t K);
 void q4k_i16_gemv(const uint8_t* W, const uint8_t* X, float* Y, size_t M, size_t K);
 
-// Q4_0 / MXFP4 mul_mat for any M: int8-MFMA GEMM for prefill shapes, GEMV otherwise.
+// Q4_0 / MXFP4
 void mul_mat_q4_0(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                   size_t M, const RowStrides& st);
 void mul_mat_mxfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                    const float* scale, float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
-// Q4_1 x Q8_1: the Q4_0 GEMM body with each block's m * s term, GEMV otherwise
+// Q4_1 x Q8_1: the GEMM is the Q4_0 body with each block's m * s term
 void mul_mat_q4_1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                   size_t M, const RowStrides& st);
 
-// IQ2_XXS mul_mat for any M: int8-MFMA GEMM for prefill shapes, GEMV otherwise.
+// IQ2_XXS
 void mul_mat_iq2_xxs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid,
                      const int8_t* signs, float* Y, size_t N, size_t K, size_t M,
                      const RowStrides& st);
-// IQ2_XS mul_mat for any M: the IQ2 GEMM with per-16 scales for prefill shapes, GEMV otherwise.
+// IQ2_XS: the IQ2 GEMM with per-16 scales
 void mul_mat_iq2_xs(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* grid, const int8_t* signs,
                     float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
 void mul_mat_iq2_xs_quantized(const uint8_t* W, const uint8_t* Xq, const int8_t* grid, const int8_t* signs,
@@ -194,11 +198,10 @@ void mul_mat_iq2_xxs_quantized(const uint8_t* W, const uint8_t* Xq, const int8_t
                                const int8_t* signs, float* Y, size_t N, size_t K, size_t M,
                                const RowStrides& st);
 
-// NVFP4 mul_mat for any M: the Q8_0 int8-MFMA GEMM for prefill shapes, GEMV otherwise
+// NVFP4: the Q8_0 GEMM body with a scale per 16 values
 void mul_mat_nvfp4(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* codebook,
                    const float* ue4m3, float* Y, size_t N, size_t K, size_t M, const RowStrides& st);
-// Q6_K / Q5_K mul_mat for any M: int8-MFMA GEMM for prefill shapes, GEMV
-// otherwise; _quantized: over an already quantized Q8_K activation.
+// Q6_K / Q5_K; _quantized: over an already quantized Q8_K activation.
 void mul_mat_q6k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
                  const RowStrides& st);
 void mul_mat_q5k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K, size_t M,
@@ -214,13 +217,12 @@ bool mul_mat_id_kq_grouped_ok(bool q6, const uint8_t* W, size_t xq_bytes, const 
 void mul_mat_id_kq_grouped(bool q6, const uint8_t* W, const uint8_t* Xq, float* Y, size_t N, size_t K,
                            const RowStrides& st, const PairArgs& pr, int n_pairs, void* ws);
 
-// Small-batch mul_mat (small_batch.hip): 2 .. kSmallBatchRows activation rows
-// on one 16-row-wide MFMA GEMM whose waves split K, any format
+// Small-batch mul_mat (small_batch.hip): several activation rows on one 16-row-wide MFMA GEMM whose waves split K, any format
 // (decode_quantized's codes, Q4_K = 8) and record alignment, K of whole
 // 256-value units.  X is quantized into Xq; _quantized reads Xq.  gemm: the
 // format's prefill GEMM takes the call too, so the faster one runs; without
 // one it takes any number of rows.  False, with nothing launched, when the
-// call does not suit it.
+// call does not suit it.  kSmallBatchRows: the most that it takes from a GEMM.
 constexpr size_t kSmallBatchRows = 64;
 bool small_batch(int fmt, const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* tab0, const void* tab1,
                  float* Y, size_t N, size_t K, size_t M, const RowStrides& st, bool gemm = true);

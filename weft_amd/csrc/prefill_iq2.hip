@@ -419,7 +419,7 @@ bool gemm_iq2_ok(const uint8_t* W, const void* Xq, const float* Y, const int8_t*
                  const int8_t* signs, size_t N, size_t K, size_t M, const RowStrides& st) {
   // MFMA path: prefill shapes with an even number of superblocks per row and
   // 4-byte aligned weight rows whose tile of 128 rows stays within 32-bit
-  // offsets; the GEMV kernels take everything else
+  // offsets; the small-batch kernel and the GEMVs take everything else
   constexpr size_t kRec = Tile<kXs>::kRec;
   const size_t ldw = N > 1 ? st.ldw : K / 256 * kRec;
   // (below 16 activation rows only when the GEMV's LDS cannot hold a row)

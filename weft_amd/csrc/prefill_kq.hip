@@ -437,7 +437,8 @@ __global__ void __launch_bounds__(kThreads, 1) kq_mfma_gemm(GemmArgs a) {
     dxq[0][lane] = bf16_split3(dxr);
   }
   // Q6_K: the terms of four superblocks, then their sum into ysum with what
-  // that addition rounds off kept in ylow.  One chain over a row of 11008 values
+  // that addition rounds off kept in ylow (all of it where the running sum is the
+  // larger one, which it is but for the first few or where it nearly cancels).  One chain over a row of 11008 values
   // had twice the error of the GEMV's short ones (against 64 bits, relative:
   // 1.3e-7, GEMV 0.70e-7; sums of eight without ylow 0.85e-7).
   v16f ysum[2] = {}, ylow[2] = {};

@@ -620,7 +620,8 @@ bool gemm_q4k_try(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_
   return true;
 }
 
-// Prefill entry: MFMA GEMM when the shape suits it, the decode GEMV otherwise.
+// Prefill entry: the small-batch kernel for a few rows, the MFMA GEMM when the
+// shape suits it, else the small-batch kernel again or the decode GEMV.
 void mul_mat_q4k(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size_t N, size_t K,
                  size_t M, const RowStrides& st) {
   if (N == 0 || M == 0 || K == 0) return;

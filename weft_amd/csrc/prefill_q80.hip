@@ -1060,7 +1060,8 @@ bool prefill_q80(const uint8_t* W, const float* X, uint8_t* Xq, const int8_t* co
   using T = WTraits<F>;
   const size_t rb = K / 32 * T::kRec;
   const size_t ldw = N > 1 ? st.ldw : rb;
-  // MFMA path preconditions; otherwise the caller runs the GEMV kernels.
+  // MFMA path preconditions; otherwise the caller runs the small-batch
+  // kernel or the GEMVs.
   // Weight rows feed dword direct-to-LDS loads (4-byte aligned) and a tile's
   // rows must stay within 32-bit offsets.
   // Below 16 activation rows the GEMV kernels run, unless their LDS cannot

@@ -1,7 +1,8 @@
 // Small-batch mul_mat: 2 .. 64 activation rows against every weight format
 // (the same products as the GEMVs and the prefill GEMMs; formats and GGML
-// line numbers in decode_staged.hip and decode_q4k.hip), and MUL_MAT_ID's
-// pairs grouped by expert at the same sizes.
+// line numbers in decode_staged.hip and decode_q4k.hip), any number of rows
+// where no prefill GEMM takes the weights, and up to 64 of MUL_MAT_ID's pairs
+// grouped by expert.
 //
 // What bounds it: one read of the weights, and the latency of that one read.
 // The GEMVs walk a batch four activation rows at a time and pay eight v_dot4
