@@ -57,7 +57,8 @@ def test_one_gemv_pass(hip, fmt, m, k, n, small):
 
 
 @pytest.mark.parametrize("fmt,m,k,n,small", [
-    ("q4_k", 32, 2048, 4096, True), ("q4_k", 32, 2048, 4097, False), ("q4_k", 17, 2304, 4097, True),
+    ("q4_k", 32, 512, 4096, True), ("q4_k", 32, 512, 4097, False), ("q4_k", 17, 768, 8192, True),
+    ("q4_k", 17, 768, 8193, False),
     ("q4_k", 33, 256, 6144, True), ("q4_k", 33, 256, 6145, False), ("q4_k", 16, 256, 13108, True),
     ("q4_k", 16, 256, 13109, False), ("mxfp4", 20, 256, 14000, True), ("mxfp4", 20, 256, 14001, False),
     ("mxfp4", 20, 3328, 12288, True), ("mxfp4", 20, 3328, 12289, False),
@@ -234,6 +235,7 @@ def test_waves_of_a_workgroup(hip, fmt, n, k, m):
     ("q4_k", 8192, 4096, 4, 1, 2, False), ("q4_k", 8192, 4096, 4, 1, 3, True),
     ("q4_k", 4096, 8192, 4, 1, 2, False), ("q4_k", 4096, 8448, 4, 1, 2, True),
     ("q4_k", 6144, 4096, 3, 1, 2, False), ("q4_k", 4096, 4096, 4, 1, 2, True),
+    ("q4_k", 14336, 2048, 4, 1, 2, False), ("q4_k", 28672, 1024, 4, 1, 2, True),
     ("nvfp4", 10240, 4096, 4, 1, 2, False), ("nvfp4", 10240, 4096, 4, 1, 3, True),
     ("nvfp4", 10240, 4096, 4, 2, 2, True), ("q5_k", 10240, 4096, 4, 1, 2, True),
 ])

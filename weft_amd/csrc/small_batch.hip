@@ -899,11 +899,11 @@ static bool small_ok(int fmt, const uint8_t* W, const uint8_t* Xq, const int8_t*
 // limits are where the two lines measured at 4096 and 11008 x 4096, 16 .. 64
 // rows, cross (MXFP4, 64 rows: 20.7 against 33.0 us at 4096 rows, 41.0 against
 // 35.3 at 11008); at 512 .. 14336 values, 16 .. 64 rows and row counts up to
-// them no call was more than 3 % slower but for two, which have limits of their
+// them no call was more than 4 % slower but for two, which have limits of their
 // own: MXFP4 past 3072 values, where a second round of workgroups is not worth
-// it (13000 x 11008, 32 rows: 65.3 against 58.1), and Q4_K at 17 .. 32 rows,
-// whose GEMM then has tiles of 32 x 64 (5632 x 512 7.0 against 6.4, 5120 x 2048
-// 9.7 against 9.1; 4096 x 2048 7.5 against 9.1, 5120 x 4096 equal).
+// it (13000 x 11008, 32 rows: 65.3 against 58.1), and Q4_K at 17 .. 32 rows of
+// 512 values, whose GEMM then has tiles of 32 x 64 (5632 x 512 7.0 against 6.4;
+// 5120 x 768 to x 4096 0 to 10 % faster here but for 1536 values, 3 % slower).
 static bool small_wins(int fmt, size_t N, size_t K, size_t M, bool gemm, bool quantize) {
   static constexpr uint8_t kFrom[9] = {3, 4, 3, 4, 2, 4, 3, 4, 2};
   static constexpr uint16_t kLimit[9] = {21000, 14000, 20000, 17000, 27000, 28000, 21000, 18000, 8192};
@@ -915,7 +915,7 @@ static bool small_wins(int fmt, size_t N, size_t K, size_t M, bool gemm, bool qu
   size_t limit = kLimit[fmt];
   if (fmt == 1 && K > 3072) limit = 12288;
   if (fmt == 8 && M > 32) limit = limit * 3 / 2;  // its GEMM is 1.5 times longer past 32 rows
-  if (fmt == 8 && M > 16 && M <= 32 && K <= 2048) limit = 4096;
+  if (fmt == 8 && M > 16 && M <= 32 && K <= 512) limit = 4096;
   // one token tile of 16 costs five eighths of one of 32
   const size_t w = M <= 16 ? N * 5 / 8 : N * ((M + 31) / 32);
   return w <= limit;
@@ -943,7 +943,8 @@ bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const i
 // 4096 values in registers (one call, experts past the Infinity Cache): 14336 x
 // 4096, 2 pairs 14.8 us against 19.7 here, 16 experts of it, 2 a token, 2 / 4 / 6
 // tokens 44 / 46 / 67 against 47 / 49 / 68, 8 tokens 83 against 75; 6144 x 8192, 8
-// experts, 2 tokens 26.5 against 29.3; 4096 x 4096 equal from 2 pairs on.  NVFP4,
+// experts, 2 tokens 26.5 against 29.3; 4096 x 4096 equal from 2 pairs on, 28672 x
+// 1024, 2 pairs 14 against 11.  NVFP4,
 // whose weights take this kernel longest, where a token has one expert: 11008 x
 // 4096, 2 / 3 pairs 21.3 / 30.6 against 25.6 / 34.2.  Of the other formats the
 // GEMV is at most as fast but for single shapes at 2 pairs.
@@ -951,7 +952,7 @@ static bool pair_gemv_wins(int fmt, size_t N, size_t K, const PairArgs& pr, int 
   const size_t values = N * K;
   const int rest = n_pairs - pr.n_ids;
   if (fmt == 5) return pr.n_ids == 1 && K > 2048 && values >= (size_t)40 << 20 && (rest == 1 || 8 * rest <= pr.n_as);
-  if (fmt != 8 || K > 8192) return false;
+  if (fmt != 8 || K < 2048 || K > 8192) return false;
   if (K > 2048 && K <= 4096 && values >= (size_t)40 << 20) return rest <= 10 && 2 * rest <= pr.n_as;
   if (values >= (size_t)32 << 20) return rest <= 3 && 4 * rest <= pr.n_as;
   return n_pairs == 2 && values >= (size_t)24 << 20;
