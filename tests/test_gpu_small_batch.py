@@ -231,10 +231,12 @@ def test_waves_of_a_workgroup(hip, fmt, n, k, m):
 
 @pytest.mark.parametrize("fmt,n,k,experts,used,m,small", [
     ("q4_k", 10240, 4096, 4, 1, 3, False), ("q4_k", 10240, 4096, 4, 1, 4, True),
-    ("q4_k", 10240, 4096, 4, 2, 2, False), ("q4_k", 10239, 4096, 4, 2, 2, True),
-    ("q4_k", 8192, 4096, 4, 1, 2, False), ("q4_k", 8192, 4096, 4, 1, 3, True),
+    ("q4_k", 10240, 4096, 8, 1, 5, False), ("q4_k", 10239, 4096, 8, 1, 5, True),
+    ("q4_k", 10239, 4096, 4, 2, 2, False),
+    ("q4_k", 8192, 4096, 4, 1, 3, False), ("q4_k", 8192, 4096, 4, 1, 4, True),
     ("q4_k", 4096, 8192, 4, 1, 2, False), ("q4_k", 4096, 8448, 4, 1, 2, True),
-    ("q4_k", 6144, 4096, 3, 1, 2, False), ("q4_k", 4096, 4096, 4, 1, 2, True),
+    ("q4_k", 6144, 4096, 3, 1, 2, False), ("q4_k", 6144, 4096, 3, 1, 3, True),
+    ("q4_k", 4096, 4096, 4, 1, 2, True),
     ("q4_k", 14336, 2048, 4, 1, 2, False), ("q4_k", 28672, 1024, 4, 1, 2, True),
     ("nvfp4", 10240, 4096, 4, 1, 2, False), ("nvfp4", 10240, 4096, 4, 1, 3, True),
     ("nvfp4", 10240, 4096, 4, 2, 2, True), ("q5_k", 10240, 4096, 4, 1, 2, True),

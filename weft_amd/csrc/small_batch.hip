@@ -943,7 +943,7 @@ bool small_batch_quantized(int fmt, const uint8_t* W, const uint8_t* Xq, const i
 // 4096 values in registers (one call, experts past the Infinity Cache): 14336 x
 // 4096, 2 pairs 14.8 us against 19.7 here, 16 experts of it, 2 a token, 2 / 4 / 6
 // tokens 44 / 46 / 67 against 47 / 49 / 68, 8 tokens 83 against 75; 6144 x 8192, 8
-// experts, 2 tokens 26.5 against 29.3; 4096 x 4096 equal from 2 pairs on, 28672 x
+// experts, 2 tokens 26.5 against 29.3, 8192 x 4096, 3 pairs of 4 14.5 and 16.2; 4096 x 4096 equal from 2 pairs on, 28672 x
 // 1024, 2 pairs 14 against 11.  NVFP4,
 // whose weights take this kernel longest, where a token has one expert: 11008 x
 // 4096, 2 / 3 pairs 21.3 / 30.6 against 25.6 / 34.2.  Of the other formats the
@@ -954,7 +954,7 @@ static bool pair_gemv_wins(int fmt, size_t N, size_t K, const PairArgs& pr, int 
   if (fmt == 5) return pr.n_ids == 1 && K > 2048 && values >= (size_t)40 << 20 && (rest == 1 || 8 * rest <= pr.n_as);
   if (fmt != 8 || K < 2048 || K > 8192) return false;
   if (K > 2048 && K <= 4096 && values >= (size_t)40 << 20) return rest <= 10 && 2 * rest <= pr.n_as;
-  if (values >= (size_t)32 << 20) return rest <= 3 && 4 * rest <= pr.n_as;
+  if (values >= (size_t)32 << 20) return rest <= 2 ? 2 * rest <= pr.n_as : rest == 3 && 4 * rest <= pr.n_as;
   return n_pairs == 2 && values >= (size_t)24 << 20;
 }
 
