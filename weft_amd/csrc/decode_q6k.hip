@@ -50,7 +50,13 @@ struct Q6Args {
 // past the Infinity Cache): 4096 x 11008 (43 superblocks, 2-byte rows) 14.1 ->
 // 11.8 us, 14336 x 4352 20.1 -> 16.3, 1024 x 14336 10.8 -> 7.1.
 // kOdd: rows that are only 2-byte aligned, so a lane's shift depends on its row.
-template <int KS, bool kOdd>
+// kMany: a row's loads all go out before the row before it is computed, which
+// pays where a wave has several rows (one call, weights past the Infinity Cache:
+// 28672 x 4096 24.4 -> 23.0 us, 14336 x 12288 36 -> 33) and costs where it has one
+// or two, or short ones (weights in it: 9856 x 1536 6.1 -> 6.5, 12288 x 2048 and
+// 6144 x 6144 5 %); kOdd rows do not
+// gain (4096 x 11008 11.6 -> 11.9).
+template <int KS, bool kOdd, bool kMany>
 __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
   constexpr int kGroups = kWaves / KS;
   extern __shared__ __align__(16) char lds[];  // Q8_K activation row, then the steps' partial sums
@@ -210,12 +216,11 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
 
   int k = 0;
   for (; k + 2 < nrows; k += 2) {
-    // (barriers: 28672 x 4096 24.6 -> 23.0 us; 4096 x 11008 11.6 -> 11.9, so not for kOdd)
     issue(bufB, k + 1);
-    if constexpr (!kOdd) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kMany) __builtin_amdgcn_sched_barrier(0);
     compute(bufA, k);
     issue(bufA, k + 2);
-    if constexpr (!kOdd) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kMany) __builtin_amdgcn_sched_barrier(0);
     compute(bufB, k + 1);
   }
   if (nrows - k == 2) {
@@ -231,13 +236,13 @@ __global__ void __launch_bounds__(kThreads) q6k_gemv_m1_kernel(Q6Args a) {
 }  // namespace
 
 namespace {
-template <bool kOdd>
+template <bool kOdd, bool kMany>
 void launch_steps(int ks, int grid, size_t lds, const Q6Args& a) {
   switch (ks) {
-    case 1: q6k_gemv_m1_kernel<1, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
-    case 2: q6k_gemv_m1_kernel<2, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
-    case 3: q6k_gemv_m1_kernel<3, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
-    default: q6k_gemv_m1_kernel<4, kOdd><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 1: q6k_gemv_m1_kernel<1, kOdd, kMany><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 2: q6k_gemv_m1_kernel<2, kOdd, kMany><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    case 3: q6k_gemv_m1_kernel<3, kOdd, kMany><<<grid, kThreads, lds, current_stream()>>>(a); break;
+    default: q6k_gemv_m1_kernel<4, kOdd, kMany><<<grid, kThreads, lds, current_stream()>>>(a); break;
   }
 }
 }  // namespace
@@ -278,9 +283,11 @@ bool decode_q6k_m1(const uint8_t* W, const float* X, uint8_t* Xq, float* Y, size
   const size_t lds = q8k_lds_row_bytes((int)K) + (ks > 1 ? 4 * (size_t)ks * a.rows_per_wg : 0);
   if (lds > max_lds_per_block()) return false;
   if (K % 512 != 0 || ldw % 4 != 0)
-    launch_steps<true>(ks, grid, lds, a);
+    launch_steps<true, false>(ks, grid, lds, a);
+  else if (K > 2048 && N >= (ks >= 3 ? 8192 : 12288))  // where the two cross, cold and warm
+    launch_steps<false, true>(ks, grid, lds, a);
   else
-    launch_steps<false>(ks, grid, lds, a);
+    launch_steps<false, false>(ks, grid, lds, a);
   check_launch("q6k_gemv_m1_kernel");
   return true;
 }
